@@ -62,7 +62,8 @@ typedef struct {
   int32_t num_work;        /* work items: (request, query tile, KV split)        */
   int32_t num_merge;       /* query tiles whose KV splits need a merge pass      */
   int32_t num_groups;      /* (request, query tile) pairs                        */
-  int32_t row_tiles;       /* 16-row MFMA tiles per work item, 1..4              */
+  int32_t row_tiles;       /* 16-row MFMA tiles per work item: 1..4, or 8 / 16 for
+                              prefill tiles (nsg_attn_plan of full query tiles)  */
   int32_t q_tile_tokens;   /* query tokens per query tile                        */
   int32_t max_splits;      /* largest KV split count of any group                */
   int32_t head_dim;

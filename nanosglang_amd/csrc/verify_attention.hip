@@ -35,7 +35,7 @@
 #include <cstdarg>
 #include <vector>
 
-#include "common.hpp"
+#include "attention.hpp"
 
 namespace nsg {
 namespace {
@@ -46,86 +46,9 @@ constexpr int kMinSplitSteps = 4;     // 32-token steps per KV split, at least
 // (~4 us) and a step of a group ~0.35 us
 constexpr int kMinGroupSteps = 8;
 constexpr int kTokIt = 32;           // KV tokens per wave step
-constexpr float kMaskVal = -1.0e30f; // finite "minus infinity" (no inf - inf)
 constexpr int64_t kHeaderBytes = 256;  // flags word + padding
 constexpr int kTargetWgPerCu = 8;
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef short v4i16 __attribute__((ext_vector_type(4)));
-typedef short v8i16 __attribute__((ext_vector_type(8)));
-
-struct AttnParams {
-  const bf16* q;
-  const bf16* kc;
-  const bf16* vc;
-  bf16* out;
-  const int* qo_indptr;
-  const int* kv_indptr;
-  const int* kv_indices;
-  const int* kv_last;
-  const int* work;
-  int num_work;
-  int Hq, Hkv, G, log2P, num_pages, causal;
-  float scale_log2;
-  int* flags;
-  float* partials;
-};
-
-__device__ __forceinline__ bf16x8 load_bf16x8(const bf16* p) {
-  u32x4 v = *reinterpret_cast<const u32x4*>(p);
-  return __builtin_bit_cast(bf16x8, v);
-}
-
-typedef float floatx2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-
-// Two floats -> packed bf16 pair (v_cvt_pk_bf16_f32, round to nearest even).
-__device__ __forceinline__ uint32_t cvt_pk_bf16(float lo, float hi) {
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(floatx2{lo, hi}, bf16x2));
-}
-
-// Transposing LDS reads of the V^T fragments, in asm.  Written through the
-// builtin, every such read after a global_load_lds gets a conservative
-// vmcnt(0) from the compiler (it cannot tell the read from the ring slots
-// still being filled), which stalls each step until every copy in flight has
-// landed; the ring's own waits (vmcnt per step plus the barrier) already
-// order these reads.  tr_issue starts the two reads of one d tile; tr_wait
-// waits until at most N LDS operations are outstanding, after which the
-// tile's registers (tied operands, so that the compiler reads them only
-// after the wait) hold the data.  LDS operations complete in order, so the
-// reads of tile dt are done once those of tile dt + 1 are the only ones left.
-__device__ __forceinline__ void tr_issue(v4i16& lo, v4i16& hi, uint32_t a0, uint32_t a1) {
-  asm volatile("ds_read_b64_tr_b16 %0, %2\n\tds_read_b64_tr_b16 %1, %3"
-               : "=&v"(lo), "=&v"(hi)
-               : "v"(a0), "v"(a1)
-               : "memory");
-}
-template <int N>
-__device__ __forceinline__ void tr_wait(v4i16& lo, v4i16& hi) {
-  asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(lo), "+v"(hi) : "n"(N) : "memory");
-}
-
-
-// LDS tile swizzles: 16-byte chunk c of token row t is stored at physical
-// chunk c ^ swz(t).  K fragments read one logical chunk of 16 consecutive
-// tokens (needs distinct banks across t).  A V^T transposing read takes one
-// 32-byte chunk pair from each of 16 rows t = 4g + j (g, j < 4): the pair
-// index is XORed with a function of t that spreads those 16 rows over every
-// 32-byte bank window (with 256-byte bank rows: 2 rows per window, the
-// minimum).
-template <int D>
-__device__ __forceinline__ int swz_k(int t) {
-  if constexpr (D == 64) return (t >> 1) & 7;  // 128-byte rows: two rows per bank cycle
-  return t & 15;                               // 256-byte rows: one row per bank cycle
-}
-template <int D>
-__device__ __forceinline__ int swz_v(int t) {
-  if constexpr (D == 64) return 2 * ((t >> 1) & 3);  // odd rows sit in the other half-row
-  return 2 * (t & 7);
-}
-
-constexpr float kLazyRescale = 8.f;  // rescale O only when a row max grows by > 2^8
 
 // LDS ring depth.  With one KV group a shallower ring lets more workgroups
 // (waves) share a CU, which hides more latency (measured: depth 3 beats 4 by
@@ -142,7 +65,6 @@ constexpr int ring_depth(int KS) { return KS == 1 ? kRingOne : kRingGroups; }
 // 160 KB of LDS (8 KB per step at head_dim 64, 16 KB at 128).
 constexpr int kv_groups_max(int D) { return D == 64 ? 4 : 2; }
 constexpr int kLdsBytes = 160 * 1024;
-constexpr int kMaxItemPages = 1024; // page ids one work item may span
 // Pages of at least 16 tokens for several KV groups: a 32-token step then
 // spans at most two pages, looked up with two scalar loads.
 constexpr int kMinGroupPage = 16;
@@ -874,6 +796,8 @@ int32_t launch_rt(const nsg_attn_plan_t* plan, const AttnParams& prm, const int*
 template <int D>
 int32_t launch_d(const nsg_attn_plan_t* plan, const AttnParams& prm, const int* merge,
                  hipStream_t stream) {
+  if ((plan->row_tiles == 8 || plan->row_tiles == 16) && plan->kv_groups == 1)
+    return launch_prefill_attn(D, plan->row_tiles / 2, plan->num_work, prm, stream);
   switch (plan->row_tiles) {
     case 1: return launch_rt<D, 1>(plan, prm, merge, stream);
     case 2: return launch_rt<D, 2>(plan, prm, merge, stream);
@@ -943,6 +867,43 @@ void fixed_capacity(int batch, int max_ql, int G, int num_kv_heads, int num_cus,
   }
   *max_work = (int)target_items(1, num_cus, num_kv_heads) + groups;
   *max_merge = groups;
+}
+
+// Rows per workgroup of the prefill kernel (prefill_attention.hip) for this
+// batch, or 0 for the verify kernel.  It does not split the KV range, so it
+// is taken when its tiles are well filled (a 256-row workgroup at least half,
+// a 128-row one three quarters) and there are enough of them: one workgroup
+// per CU, or a third of that with contexts of at most 2048 tokens.  Measured
+// (us, verify kernel -> this one): a batch of 32 prompts of 100 - 512 tokens,
+// 14 / 2 heads of 64, 42.5 -> 23.4; two prompts of 2048 - 8192, 32 / 8 heads
+// of 128, 1081 -> 609; 16 x 32 query tokens over 100 - 640, 40 -> 23.  Below
+// the line the verify kernel's KV groups and splits are ahead: one prompt of
+// 300 tokens (34 workgroups) 8.0 against 10.0, 2 x 512 tokens over 4000 -
+// 8000 (116 long workgroups) 66 against 101.
+// 256 rows only at head dim 128, where two wave groups then alternate
+// (prefill_attention.hip); at 64 the shorter 128-row workgroups were ahead
+// throughout (23.4 against 27.9 us on the 32 prompts).
+int prefill_rows(const int32_t* qo, const int32_t* kvp, int batch, int G, int num_kv_heads,
+                 int head_dim, int page_size, int num_cus) {
+  int max_pages = 0;
+  for (int b = 0; b < batch; ++b)
+    if (qo[b + 1] > qo[b]) max_pages = std::max(max_pages, kvp[b + 1] - kvp[b]);
+  if (max_pages > kMaxItemPages - 2) return 0;  // the item's page list
+  for (int rows : {256, 128}) {
+    if (rows == 256 && head_dim == 64) continue;
+    const int T = rows / G;
+    long long tiles = 0, used = 0;
+    for (int b = 0; b < batch; ++b) {
+      const int ql = qo[b + 1] - qo[b];
+      tiles += (ql + T - 1) / T;
+      used += (long long)ql * G;
+    }
+    const long long wgs = tiles * num_kv_heads;
+    const bool fills = wgs >= num_cus ||
+                       (3 * wgs >= num_cus && (long long)max_pages * page_size <= 2048);
+    if (4 * used >= (rows == 256 ? 2 : 3) * tiles * rows && fills) return rows;
+  }
+  return 0;
 }
 
 int max_splits_planned(const std::vector<int>& split_counts) {
@@ -1035,7 +996,14 @@ int32_t plan_impl(const int32_t* qo_indptr_h, const int32_t* kv_indptr_h,
   const long long t1 = target_items(1, num_cus, num_kv_heads);
   bool latency;
   int T;
-  if (fixed_work >= 0) {
+  const int prefill = fixed_work >= 0 ? 0
+                      : prefill_rows(qo_indptr_h, kv_indptr_h, batch, G, num_kv_heads, head_dim,
+                                     page_size, num_cus);
+  if (prefill) {
+    latency = false;
+    T = prefill / G;
+    if (int32_t rc = make_groups(T)) return rc;
+  } else if (fixed_work >= 0) {
     latency = page_size >= kMinGroupPage && fixed_kv_len > 0;
     T = q_tile_tokens(G, max_ql, latency);
     if (int32_t rc = make_groups(T)) return rc;
@@ -1048,7 +1016,7 @@ int32_t plan_impl(const int32_t* qo_indptr_h, const int32_t* kv_indptr_h,
       if (int32_t rc = make_groups(T)) return rc;
     }
   }
-  const int RT = (T * G + 15) / 16;
+  const int RT = prefill ? prefill / 16 : (T * G + 15) / 16;
   const int KS = latency ? kv_groups_max(head_dim) : 1;
   const long long tgt = target_items(KS, num_cus, num_kv_heads);
   long long chunk_it = std::max<long long>(
@@ -1058,6 +1026,7 @@ int32_t plan_impl(const int32_t* qo_indptr_h, const int32_t* kv_indptr_h,
       std::max<long long>(1, ((long long)(kMaxItemPages - 2) * page_size) / kTokIt);
   chunk_it = std::min(chunk_it, max_chunk_it);
   if (fixed_kv_len > 0) chunk_it = std::max<long long>(chunk_it, (fixed_kv_len + kTokIt - 1) / kTokIt);
+  if (prefill) chunk_it = max_chunk_it;  // never split (prefill_rows bounds the pages)
 
   int n = 0, max_splits = 0, n_merge = 0;
   std::vector<int> split_counts(groups.size());
@@ -1104,6 +1073,18 @@ int32_t plan_impl(const int32_t* qo_indptr_h, const int32_t* kv_indptr_h,
           if (t < reqs[r].second) order.push_back(reqs[r].first + t);
     }
   }
+  // Prefill tiles: most 64-token steps first (a counting sort), so that the
+  // last workgroups to start are short ones.
+  if (prefill) {
+    auto steps = [&](const Group& g) { return (g.kv_end + 63) / 64; };
+    int most = 0;
+    for (const Group& g : groups) most = std::max(most, steps(g));
+    std::vector<int> at((size_t)most + 2, 0);  // at[most - s]: first place of s steps
+    for (const Group& g : groups) ++at[(size_t)(most - steps(g)) + 1];
+    for (size_t i = 1; i < at.size(); ++i) at[i] += at[i - 1];
+    for (size_t gi = 0; gi < groups.size(); ++gi)
+      order[(size_t)at[(size_t)(most - steps(groups[gi]))]++] = (int)gi;
+  }
   n = 0;
   int m = 0;
   for (size_t oi = 0; oi < groups.size(); ++oi) {
@@ -1149,8 +1130,9 @@ int32_t plan_impl(const int32_t* qo_indptr_h, const int32_t* kv_indptr_h,
   plan->num_qo_heads = num_qo_heads;
   plan->num_kv_heads = num_kv_heads;
   plan->kv_groups = KS;
+  // (prefill tiles write no partials)
   plan->workspace_bytes =
-      kHeaderBytes + (int64_t)n_work * num_kv_heads * RT * 16 * (head_dim + 4) * 4;
+      kHeaderBytes + (prefill ? 0 : (int64_t)n_work * num_kv_heads * RT * 16 * (head_dim + 4) * 4);
   clear_error();
   return NSG_OK;
 }

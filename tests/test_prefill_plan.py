@@ -1,0 +1,63 @@
+"""The planner's prefill tiles (nsg_attn_plan, csrc/prefill_attention.hip): which
+batches get them, and that they cover every query row once.  Host only."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from nanosglang_amd import _native
+from nanosglang_amd._native import NSG_ATTN_WORK_INTS, AttnPlan
+
+
+def _plan(q_lens, kv_lens, Hq, Hkv, D, P=16, causal=1, cus=256):
+    lib = _native.load()
+    npg = [(L + P - 1) // P for L in kv_lens]
+    qo = np.concatenate([[0], np.cumsum(q_lens)]).astype(np.int32)
+    kvp = np.concatenate([[0], np.cumsum(npg)]).astype(np.int32)
+    last = np.asarray([(L % P) or P for L in kv_lens], np.int32)
+    cap = 1 << 16
+    work = np.zeros((cap, NSG_ATTN_WORK_INTS), np.int32)
+    pl = AttnPlan()
+    rc = lib.nsg_attn_plan(qo.ctypes.data, kvp.ctypes.data, last.ctypes.data, len(q_lens), Hq, Hkv,
+                           D, P, causal, cus, work.ctypes.data, cap, C.byref(pl))
+    assert rc == 0, lib.nsg_last_error()
+    return pl, work[:pl.num_work], qo, kvp
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,rows", [(14, 2, 64, 128), (32, 8, 128, 256), (8, 8, 64, 128),
+                                           (64, 1, 128, 256)])
+@pytest.mark.parametrize("causal", [0, 1])
+def test_tiles_cover_every_row_once_longest_first(Hq, Hkv, D, rows, causal):
+    rng = np.random.default_rng(Hq + causal)
+    kv = list(rng.integers(64, 513, 300)) + [1, 2000]
+    ql = [max(1, int(L * f)) for L, f in zip(kv, rng.choice([1.0, 0.9], len(kv)))]
+    pl, work, qo, kvp = _plan(ql, kv, Hq, Hkv, D, causal=causal)
+    G = Hq // Hkv
+    T = rows // G
+    assert (pl.row_tiles, pl.q_tile_tokens, pl.kv_groups) == (rows // 16, T, 1)
+    assert pl.num_merge == 0 and pl.max_splits == 1 and pl.workspace_bytes == 256
+    want = []
+    for b, (q, L) in enumerate(zip(ql, kv)):
+        for qb in range(0, q, T):
+            qn = min(T, q - qb)
+            end = L - q + qb + qn if causal else L
+            want.append((qo[b] + qb, qn, L - q + qb if causal else L - 1, kvp[b], 0, end, 1, 0))
+    assert sorted(map(tuple, work.tolist())) == sorted(want)
+    assert (np.diff((work[:, 5] + 63) // 64) <= 0).all()      # in 64-token steps
+
+
+@pytest.mark.parametrize("q,kv,heads,prefill", [
+    ([5] * 64, [500] * 64, (14, 2, 64), False),          # verify rows: tiles mostly padding
+    ([9] * 64, [5000] * 64, (32, 8, 128), False),
+    ([300], [300], (14, 2, 64), False),                  # too few workgroups
+    ([512] * 2, [8000] * 2, (14, 2, 64), False),         # few and long: needs the KV split
+    ([300] * 4, [300] * 4, (14, 2, 64), True),
+    ([1000], [1000], (32, 8, 128), True),
+    ([512] * 16, [8000] * 16, (14, 2, 64), True),
+    ([20000], [20000], (14, 2, 64), False),              # more pages than an item holds
+])
+def test_which_batches_get_prefill_tiles(q, kv, heads, prefill):
+    pl, _, _, _ = _plan(q, kv, *heads)
+    assert (pl.row_tiles >= 8) == prefill
+    if not prefill:      # the verify kernel's forms are what they were
+        assert pl.row_tiles <= 4 and pl.q_tile_tokens * (heads[0] // heads[1]) <= 64
