@@ -43,7 +43,7 @@ enum {
 const char* nsg_last_error(void);
 /* ABI version of this header (NSG_ABI_VERSION). */
 int32_t nsg_abi_version(void);
-#define NSG_ABI_VERSION 21
+#define NSG_ABI_VERSION 22
 
 /* ------------------------------------------------------------------------
  * Verify attention: ragged multi-query attention over the paged KV cache
@@ -440,6 +440,20 @@ int32_t nsg_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, const
 int32_t nsg_linear_fp8(const void* x, int64_t ldx, const void* w8, int64_t ldw8,
                        const float* w_scale, const void* bias, void* y, int64_t ldy, int32_t M,
                        int32_t N, int32_t K, int32_t epilogue, nsg_stream_t stream);
+
+/* The same two with device memory for fp32 partial sums, so that large weights
+ * with few output columns can split K over the GPU.  nsg_linear_workspace_bytes:
+ * the bytes (16-byte aligned, no initial contents needed) that such a split
+ * takes at this shape; 0: none is made.  With less or no workspace they are
+ * nsg_linear / nsg_linear_fp8.  Calls that share a workspace must not overlap. */
+int64_t nsg_linear_workspace_bytes(int32_t M, int32_t N, int32_t K, int32_t epilogue);
+int32_t nsg_linear_ws(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias,
+                      void* y, int64_t ldy, int32_t M, int32_t N, int32_t K, int32_t epilogue,
+                      void* workspace, int64_t workspace_bytes, nsg_stream_t stream);
+int32_t nsg_linear_fp8_ws(const void* x, int64_t ldx, const void* w8, int64_t ldw8,
+                          const float* w_scale, const void* bias, void* y, int64_t ldy, int32_t M,
+                          int32_t N, int32_t K, int32_t epilogue, void* workspace,
+                          int64_t workspace_bytes, nsg_stream_t stream);
 int32_t nsg_linear_rope_kv_fp8(const void* x, int64_t ldx, const void* w8, int64_t ldw8,
                                const float* w_scale, const void* bias, int32_t M, int32_t K,
                                int32_t num_qo_heads, int32_t num_kv_heads, int32_t head_dim,

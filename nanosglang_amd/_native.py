@@ -13,7 +13,7 @@ _PKG = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_PKG, "libnsg_spec.so")
 
 NSG_ATTN_WORK_INTS = 8
-ABI_VERSION = 21
+ABI_VERSION = 22
 
 i32, i64, u32, u64, f32 = C.c_int32, C.c_int64, C.c_uint32, C.c_uint64, C.c_float
 vp = C.c_void_p
@@ -52,6 +52,10 @@ SIGNATURES = {
     "nsg_linear_max_rows": (i32, []),
     "nsg_linear_preferred": (i32, [i32, i32, i32]),
     "nsg_linear": (i32, [vp, i64, vp, i64, vp, vp, i64, i32, i32, i32, i32, vp]),
+    "nsg_linear_workspace_bytes": (i64, [i32, i32, i32, i32]),
+    "nsg_linear_ws": (i32, [vp, i64, vp, i64, vp, vp, i64, i32, i32, i32, i32, vp, i64, vp]),
+    "nsg_linear_fp8_ws": (i32, [vp, i64, vp, i64, vp, vp, vp, i64, i32, i32, i32, i32, vp, i64,
+                                vp]),
     "nsg_linear_fp8": (i32, [vp, i64, vp, i64, vp, vp, vp, i64, i32, i32, i32, i32, vp]),
     "nsg_linear_rope_kv_fp8": (i32, [vp, i64, vp, i64, vp, vp, i32, i32, i32, i32, i32, vp, vp,
                                      vp, i32, vp, vp, vp, vp, i64, vp, vp]),

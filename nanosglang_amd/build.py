@@ -48,6 +48,7 @@ MFMA_VGPR = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
 FILE_FLAGS = {"spec_accept.hip": ["-fno-honor-nans"],
               "linear.hip": ["-Wno-inline-asm", *MFMA_VGPR],
               "lm_head.hip": ["-Wno-inline-asm", *MFMA_VGPR],
+              "ring_linear.hip": ["-Wno-inline-asm", *MFMA_VGPR],
               "verify_attention.hip": ["-fno-honor-nans", *MFMA_VGPR],
               "prefill_attention.hip": ["-fno-honor-nans", "-Wno-inline-asm", *MFMA_VGPR]}
 

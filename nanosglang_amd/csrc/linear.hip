@@ -784,6 +784,34 @@ using namespace nsg;
 constexpr int kFastRows = 160;
 constexpr int kFastRowsBig = 32;
 
+// Where ring_linear.hip takes over (both weight types alike, so that FP8 and
+// the bf16 weights it stands for agree bit for bit).  Graph replay, weights
+// cold, us, weight-streaming kernel -> ring:
+// * SwiGLU from 154 column tiles of 64 (enough workgroups for the GPU): 28672
+//   x 4096 FP8 30.3 -> 24.2 at 1 row, 39 -> 24.6 at 32, 57 -> 29.3 at 64, 108
+//   -> 58 at 160, bf16 43 -> 38 at 1 row; 22016 x 4096 FP8 24.9 -> 22.8 /
+//   47.9 -> 27.3 at 1 / 64; from 128 tiles above 32 rows (16384 x 4096: 32.9
+//   -> 27.1 at 64, but 19.6 -> 21.1 at 1; 8192 x 4096: 20.2 -> 26.4 at 64);
+// * bias, from 17 rows of weights of 24 M elements, K split: 4096 x 14336 FP8
+//   21.9 -> 16.8 at 17 rows, 34.5 -> 24.2 at 64, 63 -> 38 at 160 (14.5 ->
+//   17.6 at 16); 6144 x 4096 20.0 -> 17.3 at 64; 4096 x 4096 12.0 -> 14.8.
+constexpr int64_t kRingBiasWeight = 24ll << 20;
+constexpr int kRingBiasMinRows = 17;
+
+static bool ring_swiglu_big(int M, int N, int K) {
+  const int tiles = (N + 63) / 64;
+  return (int64_t)N * K >= kBigWeight && ring_linear_fits(M, N, K) &&
+         (tiles >= 154 || (tiles >= 128 && M > 32));
+}
+
+extern "C" int64_t nsg_linear_workspace_bytes(int32_t M, int32_t N, int32_t K,
+                                              int32_t epilogue) {
+  if (epilogue != NSG_LINEAR_BIAS || M < kRingBiasMinRows || N >= kWideN ||
+      (int64_t)N * K < kRingBiasWeight || !ring_linear_fits(M, N, K))
+    return 0;
+  return (int64_t)ring_linear_splits(N, K) * M * N * (int64_t)sizeof(float);
+}
+
 extern "C" int32_t nsg_linear_max_rows(void) { return kMaxMT * 16; }
 
 extern "C" int32_t nsg_linear_preferred(int32_t M, int32_t N, int32_t K) {
@@ -853,7 +881,8 @@ bool head_route(const LinParams& p) {
 int32_t linear_impl(const void* x, int64_t ldx, const void* w, const void* w8, int64_t ldw,
                     const float* w_scale, const void* bias, void* y, int64_t ldy, int32_t M,
                     int32_t N, int32_t K, int32_t epilogue, nsg_stream_t stream,
-                    const NormFold* nf = nullptr) {
+                    const NormFold* nf = nullptr, void* workspace = nullptr,
+                    int64_t workspace_bytes = 0) {
   NSG_CHECK_ARG(M >= 0 && N > 0 && K > 0, "M %d, N %d, K %d", M, N, K);
   if (M == 0) {
     clear_error();
@@ -893,6 +922,17 @@ int32_t linear_impl(const void* x, int64_t ldx, const void* w, const void* w8, i
   if (int32_t rc = apply_fold(p, nf, N, epilogue == NSG_LINEAR_SILU_MUL, epilogue == NSG_LINEAR_BIAS))
     return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  const bool silu = epilogue == NSG_LINEAR_SILU_MUL;
+  const int64_t ring_ws = nsg_linear_workspace_bytes(M, N, K, epilogue);
+  if (!p.sumsq_in && !p.residual && (w || (ldw % 16 == 0 && (uintptr_t)w8 % 16 == 0)) &&
+      (silu ? ring_swiglu_big(M, N, K)
+            : ring_ws > 0 && workspace && workspace_bytes >= ring_ws &&
+                  (uintptr_t)workspace % 16 == 0)) {
+    const RingLinearParams rp{p.x, w ? w : w8, p.w_scale, p.bias, p.y,
+                              static_cast<float*>(workspace), ldx, ldw, ldy, M, N, K,
+                              silu ? 1 : ring_linear_splits(N, K)};
+    return launch_ring_linear(rp, silu, s);
+  }
   if (epilogue == NSG_LINEAR_SILU_MUL && p.w && M >= kRingSwigluMinRows &&
       ring_swiglu_fits(M, N, K, p.sumsq_in ? p.sumsq_parts : 0)) {
     const GuParams gp{p.x, p.w, p.y, ldx, ldw, ldy, M, N, K,
@@ -986,6 +1026,25 @@ extern "C" int32_t nsg_linear_fp8(const void* x, int64_t ldx, const void* w8, in
                                   nsg_stream_t stream) {
   NSG_CHECK_ARG(w8 && w_scale, "null fp8 weight or scales");
   return linear_impl(x, ldx, nullptr, w8, ldw8, w_scale, bias, y, ldy, M, N, K, epilogue, stream);
+}
+
+extern "C" int32_t nsg_linear_ws(const void* x, int64_t ldx, const void* w, int64_t ldw,
+                                 const void* bias, void* y, int64_t ldy, int32_t M, int32_t N,
+                                 int32_t K, int32_t epilogue, void* workspace,
+                                 int64_t workspace_bytes, nsg_stream_t stream) {
+  NSG_CHECK_ARG(w, "null weight");
+  return linear_impl(x, ldx, w, nullptr, ldw, nullptr, bias, y, ldy, M, N, K, epilogue, stream,
+                     nullptr, workspace, workspace_bytes);
+}
+
+extern "C" int32_t nsg_linear_fp8_ws(const void* x, int64_t ldx, const void* w8, int64_t ldw8,
+                                     const float* w_scale, const void* bias, void* y, int64_t ldy,
+                                     int32_t M, int32_t N, int32_t K, int32_t epilogue,
+                                     void* workspace, int64_t workspace_bytes,
+                                     nsg_stream_t stream) {
+  NSG_CHECK_ARG(w8 && w_scale, "null fp8 weight or scales");
+  return linear_impl(x, ldx, nullptr, w8, ldw8, w_scale, bias, y, ldy, M, N, K, epilogue, stream,
+                     nullptr, workspace, workspace_bytes);
 }
 
 extern "C" int32_t nsg_linear_rope_kv(const void* x, int64_t ldx, const void* w, int64_t ldw,

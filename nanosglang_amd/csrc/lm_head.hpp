@@ -69,4 +69,24 @@ struct GuParams {
 bool ring_swiglu_fits(int M, int N, int K, int parts);
 int32_t launch_ring_swiglu(const GuParams& p, hipStream_t s);
 
+// 8B-class linear layers (ring_linear.hip): y = x W^T + bias, or SwiGLU (W:
+// the gate rows, then the up rows; no bias).  w_scale set: W
+// holds e4m3fn bytes with one scale per row (ldw in elements either way).
+// splits > 1 (bias only): K is split over that many workgroups per column
+// tile, whose fp32 partials ([splits][M][N]) go through the caller's memory.
+constexpr int kRlMaxSplits = 8;
+struct RingLinearParams {
+  const bf16* x;
+  const void* w;
+  const float* w_scale;
+  const bf16* bias;
+  bf16* y;
+  float* partials;
+  int64_t ldx, ldw, ldy;
+  int M, N, K, splits;
+};
+bool ring_linear_fits(int M, int N, int K);
+int ring_linear_splits(int N, int K);
+int32_t launch_ring_linear(const RingLinearParams& p, bool silu, hipStream_t s);
+
 }  // namespace nsg

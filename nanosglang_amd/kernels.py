@@ -876,6 +876,7 @@ def silu_mul(gate_up: torch.Tensor, out: torch.Tensor | None = None) -> torch.Te
 
 
 LINEAR_BIAS, LINEAR_SILU_MUL = 0, 1
+SPLIT_K_MIN_WEIGHT = 16 << 20    # weights from which nsg_linear_workspace_bytes may be non-zero
 FP8 = torch.float8_e4m3fn
 
 
@@ -989,6 +990,23 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
     if out is None:
         out = torch.empty(M, N, dtype=torch.bfloat16, device=x.device)
     epi = LINEAR_SILU_MUL if swiglu else LINEAR_BIAS
+    # large weights with few columns split K through fp32 partials: the
+    # caching allocator's memory, ordered with this stream's other work
+    need = 0 if swiglu or N * K < SPLIT_K_MIN_WEIGHT else \
+        lib.nsg_linear_workspace_bytes(M, N, K, epi)
+    if need > 0:
+        ws = torch.empty(need, dtype=torch.uint8, device=x.device)
+        if fp8:
+            check(lib.nsg_linear_fp8_ws(
+                x.data_ptr(), x.stride(0), weight.data_ptr(), weight.stride(0),
+                w_scale.data_ptr(), _ptr(bias), out.data_ptr(), out.stride(0), M, N, K, epi,
+                ws.data_ptr(), need, _stream_ptr(x.device)), "nsg_linear_fp8_ws")
+        else:
+            check(lib.nsg_linear_ws(
+                x.data_ptr(), x.stride(0), weight.data_ptr(), weight.stride(0), _ptr(bias),
+                out.data_ptr(), out.stride(0), M, N, K, epi, ws.data_ptr(), need,
+                _stream_ptr(x.device)), "nsg_linear_ws")
+        return out
     if fp8:
         check(lib.nsg_linear_fp8(x.data_ptr(), x.stride(0), weight.data_ptr(), weight.stride(0),
                                  w_scale.data_ptr(), _ptr(bias), out.data_ptr(), out.stride(0),
