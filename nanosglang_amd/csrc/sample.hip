@@ -89,6 +89,7 @@ struct SmpParams {
   uint32_t* hcnt;     // [rows][kMaxStages][256]
   u64* hmass;         // [rows][kMaxStages][256]
   SmpState* st;       // [rows][kMaxStages + 1]
+  uint32_t* todo;     // [rows]: 1 for a row left to the staged launches; null: all rows
   u64* csum;          // [rows][nch]
   uint32_t* ceq;      // [rows][nch]
 };
@@ -313,6 +314,7 @@ __device__ SmpState state_before(const SmpParams& p, int row, int s, bool store,
 template <typename T>
 __global__ __launch_bounds__(kSThreads) void max_kernel(SmpParams p, bool vec) {
   const int ch = blockIdx.x, row = blockIdx.y, tid = threadIdx.x;
+  if (p.todo && p.todo[row] == 0) return;
   const int nst = p.nk + p.np;
   for (int i = ch * kSThreads + tid; i < nst * kBins; i += p.nch * kSThreads) {
     p.hcnt[(int64_t)row * kMaxStages * kBins + i] = 0;
@@ -362,6 +364,7 @@ __global__ __launch_bounds__(kSThreads) void hist_kernel(SmpParams p, int s, boo
   constexpr int kCopies = 4;  // per wave, by lane & 3: a quarter of the same-bin conflicts
   typedef typename std::conditional<kCount, uint32_t, u64>::type H;
   const int ch = blockIdx.x, row = blockIdx.y, tid = threadIdx.x;
+  if (p.todo && p.todo[row] == 0) return;
   const int lane = tid & 63, wave = tid >> 6;
   __shared__ H lh[kSWaves * kCopies][kBins];
   __shared__ SmpState s_st;
@@ -430,6 +433,7 @@ __global__ __launch_bounds__(kSThreads) void hist_kernel(SmpParams p, int s, boo
 template <typename T>
 __global__ __launch_bounds__(kSThreads) void sums_kernel(SmpParams p, bool vec) {
   const int ch = blockIdx.x, row = blockIdx.y, tid = threadIdx.x;
+  if (p.todo && p.todo[row] == 0) return;
   const int lane = tid & 63, wave = tid >> 6;
   __shared__ SmpState s_st;
   __shared__ float s_mc;
@@ -518,6 +522,7 @@ __device__ u64 block_excl_scan_u64(u64 x, u64* sh, u64* total) {
 template <typename T>
 __global__ __launch_bounds__(kSThreads) void select_kernel(SmpParams p, bool vec) {
   const int row = blockIdx.x, tid = threadIdx.x;
+  if (p.todo && p.todo[row] == 0) return;
   const int lane = tid & 63, wave = tid >> 6;
   __shared__ u64 sh[kSWaves];
   __shared__ int s_ch;
@@ -651,9 +656,457 @@ __global__ __launch_bounds__(kSThreads) void select_kernel(SmpParams p, bool vec
   if (tid == 0) p.out[row] = s_tok;
 }
 
+// ---- top-k draws (with or without top-p) of K <= kTkMaxK: one launch ----
+// A row's K-th largest logit needs no histogram of the whole row: K of the
+// largest logits lie above the smallest of 16 numbers, wave w's ceil(K / 16)-th
+// largest lane maximum.  So one workgroup per row (1024 threads) reads the
+// row once -- bf16 rows of up to 155,648 logits stay in registers, longer and
+// fp32 rows are read a second time, from L2 --, collects the few hundred
+// logits at or above that bound in LDS, and evaluates the rule on them: the
+// K-th largest key by radix selection, then, over the tokens kept by top-k,
+// each one's mass above it (top-p) and its mass prefix in vocabulary order (the
+// draw), by direct sums of the same 2^-40 integers as the staged launches, so
+// the token is the same.  The staged form took a launch per key byte and
+// filter and three more, 7 - 10 us each whatever its work.  Eager calls, us,
+// staged -> this: 32 rows x 151,936 bf16, top-k 50 and top-p 0.9 57.2 -> 28.5,
+// top-k alone 41.3 -> 23.7, fp32 83 -> 41 / 56 -> 32; 32 x 32,000 bf16 41 -> 27;
+// top-k 200 and top-p 0.95 57 -> 39 (the sums over kept tokens grow with K^2:
+// the line lies at 256, where both forms are level).  About 10 us of that are
+// the marked rows' launches, which return at once.
+// Rows with so many ties that the lists overflow (more than 8192 logits at the
+// bound, or 1024 kept) are marked (todo), and the staged launches that follow do
+// those rows only: every other row's workgroups return at once.
+constexpr int kTkThreads = 1024;
+constexpr int kTkWaves = kTkThreads / 64;
+constexpr int kTkMaxK = 256;
+constexpr int kTkSlotCap = 2048;  // slots of 8 logits that hold one to collect
+constexpr int kTkCap = 8192;   // collected logits
+constexpr int kTkKeep = 1024;  // tokens kept by top-k
+constexpr int kTkSlots = 19;   // slots of 8 bf16 logits a thread holds
+
+typedef short v2i16 __attribute__((ext_vector_type(2)));
+
+// Signed order-preserving integers of raw logit bits (-0 is -1 until
+// tk_key): missing elements (all bits set) are the lowest.
+template <typename T>
+struct TkBits;
+template <>
+struct TkBits<bf16> {
+  static constexpr int kDwords = 4;  // of 8 elements
+  static __device__ __forceinline__ uint32_t order(uint32_t packed) {
+    v2i16 x = __builtin_bit_cast(v2i16, packed);
+    x ^= (x >> 15) & (short)0x7FFF;
+    return __builtin_bit_cast(uint32_t, x);
+  }
+  static __device__ __forceinline__ int at(const uint32_t* d, int i) {  // i unrolled
+    return (int)(short)(i & 1 ? d[i >> 1] >> 16 : d[i >> 1] & 0xFFFFu);
+  }
+  static __device__ __forceinline__ int max8(const uint32_t* d) {
+    v2i16 m = __builtin_bit_cast(v2i16, d[0]);
+#pragma unroll
+    for (int i = 1; i < 4; ++i)
+      m = __builtin_elementwise_max(m, __builtin_bit_cast(v2i16, d[i]));
+    return max((int)m[0], (int)m[1]);
+  }
+};
+template <>
+struct TkBits<float> {
+  static constexpr int kDwords = 8;
+  static __device__ __forceinline__ uint32_t order(uint32_t b) {
+    return b ^ ((uint32_t)((int)b >> 31) & 0x7FFFFFFFu);
+  }
+  static __device__ __forceinline__ int at(const uint32_t* d, int i) { return (int)d[i]; }
+  static __device__ __forceinline__ int max8(const uint32_t* d) {
+    int m = (int)d[0];
+#pragma unroll
+    for (int i = 1; i < 8; ++i) m = max(m, (int)d[i]);
+    return m;
+  }
+};
+// SKey's unsigned key of an order integer.
+template <typename T>
+__device__ __forceinline__ uint32_t tk_key(int order) {
+  if (order == -1) order = 0;  // -0 == +0
+  return (uint32_t)order + (SKey<T>::kBits == 16 ? 0x8000u : 0x80000000u);
+}
+
+// A row in slots of 8 elements: slot s holds elements head - 8 + 8 s .. + 8,
+// head (1 .. 8) chosen so that whole slots are 16-byte aligned whatever the
+// row's address; the elements outside the row (of the first and the last
+// slot) are missing.
+template <typename T>
+struct TkRow {
+  const T* x;
+  int V, head, slots;
+  __device__ __forceinline__ TkRow(const SmpParams& p, int row) {
+    x = reinterpret_cast<const T*>(row_ptr<T>(p, row));
+    V = p.V;
+    head = (int)((0u - (uint32_t)reinterpret_cast<uintptr_t>(x)) % 16u / sizeof(T));
+    if (head == 0) head = 8;
+    slots = 1 + (max(V - head, 0) + 7) / 8;
+  }
+  __device__ __forceinline__ int first(int s) const { return head - 8 + 8 * s; }
+  // raw bits, packed as they lie in memory
+  __device__ __forceinline__ void load(int s, uint32_t* d) const {
+    const int e0 = first(s);
+    if (e0 >= 0 && e0 + 8 <= V) {
+#pragma unroll
+      for (int i = 0; i < TkBits<T>::kDwords; i += 4) {
+        const u32x4 v = *reinterpret_cast<const u32x4*>(x + e0 + i * (4 / sizeof(T)));
+#pragma unroll
+        for (int k = 0; k < 4; ++k) d[i + k] = v[k];
+      }
+      return;
+    }
+#pragma unroll
+    for (int i = 0; i < TkBits<T>::kDwords; ++i) d[i] = 0xFFFFFFFFu;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if (e0 + i < 0 || e0 + i >= V) continue;
+      if constexpr (sizeof(T) == 2) {
+        const uint32_t b = reinterpret_cast<const uint16_t*>(x)[e0 + i];
+        d[i >> 1] = i & 1 ? (d[i >> 1] & 0xFFFFu) | (b << 16) : (d[i >> 1] & 0xFFFF0000u) | b;
+      } else {
+        d[i] = reinterpret_cast<const uint32_t*>(x)[e0 + i];
+      }
+    }
+  }
+  __device__ __forceinline__ void load_ordered(int s, uint32_t* d) const {
+    load(s, d);
+#pragma unroll
+    for (int i = 0; i < TkBits<T>::kDwords; ++i) d[i] = TkBits<T>::order(d[i]);
+  }
+};
+
+template <typename T, bool HELD>
+__global__ __launch_bounds__(kTkThreads) void topk_kernel(SmpParams p) {
+  constexpr int DW = TkBits<T>::kDwords;
+  constexpr int kBatch = 4;  // slots in flight when the row is not held
+  __shared__ __attribute__((aligned(16))) uint32_t s_key[kTkCap], s_idx[kTkCap];
+  __shared__ __attribute__((aligned(16))) u64 s_w[kTkKeep];
+  __shared__ __attribute__((aligned(16))) uint32_t s_raw[kTkSlotCap][DW];
+  __shared__ uint32_t s_slot[kTkSlotCap];
+  __shared__ uint32_t s_hist[kBins];
+  __shared__ uint32_t s_wmax[kTkWaves], s_wthr[kTkWaves];
+  __shared__ uint32_t s_n, s_ns, s_n2, s_bin, s_above;
+  const int row = blockIdx.x, tid = threadIdx.x;
+  const int lane = tid & 63, wave = tid >> 6;
+  const TkRow<T> r(p, row);
+  if (tid == 0) p.todo[row] = 0;
+  const float u = p.u[(int64_t)row * p.u_stride];  // (used last: lands meanwhile)
+
+  // ---- the row, and each thread's largest logit ----
+  constexpr int kMissing = SKey<T>::kBits == 16 ? -32768 : INT_MIN;
+  uint32_t held[HELD ? kTkSlots : 1][DW];
+  int mx = kMissing;
+  if constexpr (HELD) {
+#pragma unroll
+    for (int j = 0; j < kTkSlots; ++j) {
+      if (j * kTkThreads < r.slots) {  // wave-uniform
+        if (tid + j * kTkThreads < r.slots) {
+          r.load(tid + j * kTkThreads, held[j]);
+        } else {
+#pragma unroll
+          for (int i = 0; i < DW; ++i) held[j][i] = 0xFFFFFFFFu;
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < kTkSlots; ++j) {
+      if (j * kTkThreads < r.slots) {
+#pragma unroll
+        for (int i = 0; i < DW; ++i) held[j][i] = TkBits<T>::order(held[j][i]);
+        mx = max(mx, TkBits<T>::max8(held[j]));
+      }
+    }
+  } else {
+    for (int s0 = tid; s0 < r.slots; s0 += kBatch * kTkThreads) {
+      uint32_t d[kBatch][DW];
+#pragma unroll
+      for (int b = 0; b < kBatch; ++b) r.load(min(s0 + b * kTkThreads, r.slots - 1), d[b]);
+#pragma unroll
+      for (int b = 0; b < kBatch; ++b) {
+        if (s0 + b * kTkThreads >= r.slots) break;  // each slot counts for one thread only
+#pragma unroll
+        for (int i = 0; i < DW; ++i) d[b][i] = TkBits<T>::order(d[b][i]);
+        mx = max(mx, TkBits<T>::max8(d[b]));
+      }
+    }
+  }
+
+  // ---- row maximum, and a bound with at least K logits at or above it ----
+  const uint32_t mk = tk_key<T>(mx);
+  {
+    uint32_t wm = mk;
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) wm = max(wm, (uint32_t)__shfl_xor((int)wm, o, 64));
+    const int m = (p.K + kTkWaves - 1) / kTkWaves;  // 1 .. 16
+    uint32_t t = 0;  // the wave's m-th largest lane maximum
+    for (int b = SKey<T>::kBits - 1; b >= 0; --b) {
+      const uint32_t c = t | (1u << b);
+      if (__builtin_popcountll(__builtin_amdgcn_ballot_w64(mk >= c)) >= m) t = c;
+    }
+    if (lane == 0) {
+      s_wmax[wave] = wm;
+      s_wthr[wave] = t;
+    }
+    if (tid == 0) s_n = s_ns = s_n2 = 0;
+  }
+  __syncthreads();
+  uint32_t maxkey = 0, bound = 0xFFFFFFFFu;
+#pragma unroll
+  for (int w = 0; w < kTkWaves; ++w) {
+    maxkey = max(maxkey, s_wmax[w]);
+    bound = min(bound, s_wthr[w]);
+  }
+  const float mc = max_c<T>(p, maxkey);
+  auto weight = [&](uint32_t key) {
+    return weight_of(SKey<T>::val(SKey<T>::bits_of_key(key)), p.c, mc);
+  };
+  const u64 wmax = weight(maxkey);  // 2^40 up to the rounding of max * c
+  if (wmax == 0) {  // no positive weight (an infinite or NaN maximum)
+    if (tid == 0) p.out[row] = -1;
+    return;
+  }
+  if (wmax > 1ull << 41) {  // that rounding is no longer small: sums might wrap
+    if (tid == 0) p.todo[row] = 1;
+    return;
+  }
+
+  // ---- collect the logits at or above the bound: first the slots that hold
+  //      any (places by ballots, one counter update per wave), then, a thread
+  //      per element of those, the logits ----
+  auto collect = [&](uint32_t key0) {
+    const int o0 = (int)(key0 - (SKey<T>::kBits == 16 ? 0x8000u : 0x80000000u));
+    const int thr = o0 == 0 ? -1 : o0;  // both zeros
+    auto place = [&](uint32_t* counter, uint32_t count) {  // wave-uniform count > 0
+      uint32_t at = 0;
+      if (lane == 0) at = atomicAdd(counter, count);
+      return (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
+    };
+    auto below = [&](uint64_t bits) {  // bits of lanes before this one
+      return __builtin_amdgcn_mbcnt_hi((uint32_t)(bits >> 32),
+                                       __builtin_amdgcn_mbcnt_lo((uint32_t)bits, 0u));
+    };
+    auto keep_slots = [&](auto n_slots, int s_first, auto&& data) {  // slots s_first + 1024 j
+      constexpr int N = decltype(n_slots)::value;
+      uint64_t hit[N];
+      uint32_t count = 0;
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        const bool in = s_first + j * kTkThreads < r.slots;
+        hit[j] = __builtin_amdgcn_ballot_w64(in && TkBits<T>::max8(data(j)) >= thr);
+        count += (uint32_t)__builtin_popcountll(hit[j]);
+      }
+      if (count == 0) return;
+      uint32_t at = place(&s_ns, count);
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        if (hit[j] == 0) continue;
+        const uint32_t mine = at + below(hit[j]);
+        if ((hit[j] >> lane & 1) && mine < kTkSlotCap) {
+          s_slot[mine] = (uint32_t)(s_first + j * kTkThreads);
+#pragma unroll
+          for (int i = 0; i < DW; i += 4)
+            *reinterpret_cast<u32x4*>(&s_raw[mine][i]) =
+                u32x4{data(j)[i], data(j)[i + 1], data(j)[i + 2], data(j)[i + 3]};
+        }
+        at += (uint32_t)__builtin_popcountll(hit[j]);
+      }
+    };
+    if constexpr (HELD) {
+      keep_slots(std::integral_constant<int, kTkSlots>{}, tid,
+                 [&](int j) -> const uint32_t* { return held[j]; });
+    } else {
+      for (int s0 = tid; s0 - tid < r.slots; s0 += kBatch * kTkThreads) {
+        uint32_t d[kBatch][DW];
+#pragma unroll
+        for (int b = 0; b < kBatch; ++b)
+          r.load_ordered(min(s0 + b * kTkThreads, r.slots - 1), d[b]);
+        keep_slots(std::integral_constant<int, kBatch>{}, s0,
+                   [&](int j) -> const uint32_t* { return d[j]; });
+      }
+    }
+    __syncthreads();
+    const int elems = 8 * (int)min(s_ns, (uint32_t)kTkSlotCap);
+    for (int q0 = wave * 64; q0 < elems; q0 += kTkThreads) {
+      const int q = q0 + lane;
+      const int sl = min(q, elems - 1) >> 3;
+      const int i = q & 7;
+      int o;
+      if constexpr (sizeof(T) == 2) {
+        const uint32_t d = s_raw[sl][i >> 1];
+        o = (int)(short)(i & 1 ? d >> 16 : d & 0xFFFFu);
+      } else {
+        o = (int)s_raw[sl][i];
+      }
+      const int e = r.first((int)s_slot[sl]) + i;
+      const uint64_t hit =
+          __builtin_amdgcn_ballot_w64(q < elems && o >= thr && e >= 0 && e < r.V);
+      if (hit == 0) continue;
+      const uint32_t at = place(&s_n, (uint32_t)__builtin_popcountll(hit)) + below(hit);
+      if ((hit >> lane & 1) && at < kTkCap) {
+        s_key[at] = tk_key<T>(o);
+        s_idx[at] = (uint32_t)e;
+      }
+    }
+    __syncthreads();
+  };
+  collect(bound);
+  if (s_ns > kTkSlotCap || s_n > kTkCap) {
+    // leave out what has no weight (masked logits): a key whose exponent is
+    // below -41 weighs less than 2^-40
+    uint32_t lo = 0, hi = maxkey;
+    while (hi - lo > 1) {
+      const uint32_t mid = lo + (hi - lo) / 2;
+      const float v = SKey<T>::val(SKey<T>::bits_of_key(mid));
+      if (__builtin_fmaf(v, p.c, -mc) >= -41.f) hi = mid;
+      else lo = mid;
+    }
+    __syncthreads();
+    if (tid == 0) s_n = s_ns = 0;
+    __syncthreads();
+    collect(max(bound, hi));
+    if (s_ns > kTkSlotCap || s_n > kTkCap) {
+      if (tid == 0) p.todo[row] = 1;
+      return;
+    }
+  }
+  const int n = (int)s_n;
+
+  // ---- the K-th largest key (fewer than K collected: all are kept) ----
+  uint32_t tk = 0;
+  if (n > p.K) {
+    uint32_t need = (uint32_t)p.K;
+    for (int shift = SKey<T>::kBits - 8; shift >= 0; shift -= 8) {
+      if (tid < kBins) s_hist[tid] = 0;
+      __syncthreads();
+      for (int i = tid; i < n; i += kTkThreads) {
+        const uint32_t k = s_key[i];
+        if (shift == SKey<T>::kBits - 8 || (k >> (shift + 8)) == tk)
+          atomicAdd(&s_hist[(k >> shift) & 0xFFu], 1u);
+      }
+      __syncthreads();
+      if (wave == 0) {
+        uint32_t h[4], sum = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sum += h[j] = s_hist[4 * lane + j];
+        uint32_t incl = sum;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+          const uint32_t y = __shfl_up(incl, o, 64);
+          if (lane >= o) incl += y;
+        }
+        uint32_t above = __shfl(incl, 63, 64) - incl;  // in bins above this lane's
+        const uint64_t reach = __builtin_amdgcn_ballot_w64(above + sum >= need);
+        if (lane == 63 - __builtin_clzll(reach)) {  // the highest lane that reaches (one does)
+          int j = 3;
+          while (j > 0 && above + h[j] < need) above += h[j--];
+          s_bin = 4 * lane + j;
+          s_above = above;
+        }
+      }
+      __syncthreads();
+      tk = (tk << 8) | s_bin;
+      need -= s_above;
+    }
+  }
+
+  // ---- the tokens kept by top-k, in place at the front of the lists ----
+  uint32_t ck[kTkCap / kTkThreads], ci[kTkCap / kTkThreads];
+#pragma unroll
+  for (int j = 0; j < kTkCap / kTkThreads; ++j) {
+    const int i = tid + j * kTkThreads;
+    ck[j] = i < n ? s_key[i] : 0u;
+    ci[j] = i < n ? s_idx[i] : 0u;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < kTkCap / kTkThreads; ++j) {
+    if (tid + j * kTkThreads < n && ck[j] >= tk) {
+      const uint32_t at = atomicAdd(&s_n2, 1u);
+      if (at < kTkKeep) {
+        s_key[at] = ck[j];
+        s_idx[at] = ci[j];
+        s_w[at] = weight(ck[j]);
+      }
+    }
+  }
+  __syncthreads();
+  const int n2 = (int)s_n2;
+  if (n2 > kTkKeep) {
+    if (tid == 0) p.todo[row] = 1;
+    return;
+  }
+  __syncthreads();  // (s_n2 is read before anything below)
+
+  // The sums over the kept tokens: 2^lg threads per token (adjacent lanes),
+  // each a share of the tokens, so that every thread works on a few terms.
+  int lg = 0;
+  while (lg < 6 && n2 << (lg + 1) <= kTkThreads) ++lg;
+  const int tok = tid >> lg, part = tid & ((1 << lg) - 1), step = 1 << lg;
+  uint32_t key = 0, idx = 0;
+  u64 w = 0;
+  if (tok < n2) {
+    key = s_key[tok];
+    idx = s_idx[tok];
+    w = s_w[tok];
+  }
+  auto group_sum = [&](u64 v) {
+    for (int o = 1; o < step; o <<= 1)
+      v += ((u64)(uint32_t)__shfl_xor((int)(uint32_t)(v >> 32), o, 64) << 32) +
+           (uint32_t)__shfl_xor((int)(uint32_t)v, o, 64);
+    return v;
+  };
+
+  // ---- top-p: a token stays while the mass before it, in order of falling
+  //      key, then index, is below top_p Z ----
+  if (p.P < 1.0) {
+    u64 z = 0, above = 0;
+    if (tok < n2) {
+#pragma unroll 4
+      for (int j = part; j < n2; j += step) {
+        const uint32_t kj = s_key[j];
+        const u64 wj = s_w[j];
+        z += wj;
+        // (a tie weighs the same: the ties before this token as mass too)
+        above += kj > key || (kj == key && s_idx[j] < idx) ? wj : 0;
+      }
+    }
+    z = group_sum(z);
+    above = group_sum(above);
+    __syncthreads();
+    if (tok < n2) {
+      if (!((double)above < p.P * (double)z)) w = 0;
+      if (part == 0) s_w[tok] = w;
+    }
+    __syncthreads();
+  }
+
+  // ---- the draw: inverse CDF in vocabulary order ----
+  u64 z = 0, pre = 0;
+  if (tok < n2) {
+#pragma unroll 4
+    for (int j = part; j < n2; j += step) {
+      const u64 wj = s_w[j];
+      z += wj;
+      pre += s_idx[j] < idx ? wj : 0;
+    }
+  }
+  z = group_sum(z);
+  pre = group_sum(pre);
+  if (tok < n2 && part == 0) {
+    u64 target = (u64)((double)u * (double)z);
+    if (target >= z) target = z - 1;  // (z > 0: the largest logit is kept)
+    if (w > 0 && pre <= target && target < pre + w) p.out[row] = idx;
+  }
+}
+
 struct SLayout {
   int nch, cs;
-  int64_t cmax_off, hcnt_off, hmass_off, st_off, csum_off, ceq_off, total;
+  int64_t cmax_off, hcnt_off, hmass_off, st_off, csum_off, ceq_off;
+  int64_t staged;  // bytes of the staged launches; then the row marks of topk_kernel
+  int64_t total;
 };
 
 SLayout slayout(int rows, int V) {
@@ -669,12 +1122,21 @@ SLayout slayout(int rows, int V) {
   L.st_off = L.hmass_off + al((int64_t)rows * kMaxStages * kBins * 8);
   L.csum_off = L.st_off + al((int64_t)rows * (kMaxStages + 1) * sizeof(SmpState));
   L.ceq_off = L.csum_off + al((int64_t)rows * kSMaxChunks * 8);
-  L.total = L.ceq_off + al((int64_t)rows * kSMaxChunks * 4);
+  L.staged = L.ceq_off + al((int64_t)rows * kSMaxChunks * 4);
+  L.total = L.staged + al((int64_t)rows * 4);
   return L;
 }
 
 template <typename T>
 int32_t launch_sample(const SmpParams& p, bool vec, hipStream_t s) {
+  if (p.todo) {
+    // (a bf16 row of 8 head elements at most and whole slots after them)
+    if (sizeof(T) == 2 && p.V <= 8 * (kTkThreads * kTkSlots - 1))
+      hipLaunchKernelGGL((topk_kernel<T, sizeof(T) == 2>), dim3(p.rows), dim3(kTkThreads), 0, s, p);
+    else
+      hipLaunchKernelGGL((topk_kernel<T, false>), dim3(p.rows), dim3(kTkThreads), 0, s, p);
+    if (int32_t rc = launch_status("sample topk_kernel")) return rc;
+  }
   const dim3 g(p.nch, p.rows);
   hipLaunchKernelGGL((max_kernel<T>), g, dim3(kSThreads), 0, s, p, vec);
   int32_t rc = launch_status("sample max_kernel");
@@ -726,9 +1188,9 @@ extern "C" int32_t nsg_sample(const void* logits, int64_t row_stride, int32_t lo
   NSG_CHECK_ARG(greedy || uniforms, "uniforms required when temperature > 0");
   NSG_CHECK_ARG(row_stride >= vocab, "row_stride %lld < vocab %d", (long long)row_stride, vocab);
   const SLayout L = slayout(rows, vocab);
-  if (workspace_bytes < L.total) {
+  if (workspace_bytes < L.staged) {
     set_error("workspace has %lld bytes, needs %lld", (long long)workspace_bytes,
-              (long long)L.total);
+              (long long)L.staged);
     return NSG_ERR_WORKSPACE;
   }
   SmpParams p{};
@@ -756,6 +1218,10 @@ extern "C" int32_t nsg_sample(const void* logits, int64_t row_stride, int32_t lo
   p.st = reinterpret_cast<SmpState*>(ws + L.st_off);
   p.csum = reinterpret_cast<u64*>(ws + L.csum_off);
   p.ceq = reinterpret_cast<uint32_t*>(ws + L.ceq_off);
+  // (a workspace without room for the marks: the staged launches alone)
+  p.todo = p.K > 0 && p.K <= kTkMaxK && workspace_bytes >= L.total
+               ? reinterpret_cast<uint32_t*>(ws + L.staged)
+               : nullptr;
   const bool vec = (reinterpret_cast<uintptr_t>(logits) % 16 == 0) &&
                    ((row_stride * esz) % 16 == 0);
   hipStream_t s = static_cast<hipStream_t>(stream);
