@@ -1102,14 +1102,18 @@ int32_t plan_impl(const int32_t* qo_indptr_h, const int32_t* kv_indptr_h,
       w[4] = w[5] = w[6] = w[7] = 0;
       ++m;
     }
+    // even shares of the group's steps (each at most chunk_it): with whole
+    // chunks and a short rest the last wave of workgroups ends unevenly
+    // (large shape, three draws of lengths: 308 / 302 / 298 -> 299 / 294 / 292 us)
+    const long long its = (g.kv_end + kTokIt - 1) / kTokIt;
     for (int s = 0; s < ns; ++s) {
       int32_t* w = work_h + (size_t)n * NSG_ATTN_WORK_INTS;
       w[0] = qs;
       w[1] = g.qn;
       w[2] = g.lim0;
       w[3] = kv_indptr_h[g.b];
-      w[4] = (int)(s * chunk_it * kTokIt);
-      w[5] = (int)std::min<long long>(g.kv_end, (s + 1) * chunk_it * kTokIt);
+      w[4] = (int)(its * s / ns * kTokIt);
+      w[5] = (int)std::min<long long>(g.kv_end, its * (s + 1) / ns * kTokIt);
       w[6] = ns;
       w[7] = 0;
       ++n;
