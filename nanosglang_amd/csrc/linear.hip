@@ -1106,7 +1106,9 @@ extern "C" int32_t nsg_linear_rope_kv_fold(
 // ---- lm_head + greedy token: argmax of the bf16 logits, never stored ----
 extern "C" int64_t nsg_linear_argmax_workspace_bytes(int32_t M, int32_t N) {
   if (M <= 0 || N <= 0) return 0;
-  return (int64_t)M * ((N + 15) / 16) * (int64_t)sizeof(uint64_t);
+  // a key per 16 columns, and per column group of the lm_head kernel (up to 4
+  // in a single 128-column tile)
+  return (int64_t)M * std::max(4, (N + 15) / 16) * (int64_t)sizeof(uint64_t);
 }
 
 extern "C" int32_t nsg_linear_argmax(const void* x, int64_t ldx, const void* w, int64_t ldw,

@@ -7,19 +7,16 @@
 // group (linear.hip) re-reads it five times through the caches, and one that
 // re-reads x per 16-column tile moves x's 287 KB thousands of times.  Here:
 //
-// * a persistent workgroup per CU walks its column tiles (128 output columns:
-//   4 waves x 2 W tiles of 16) and, per tile, K in 64-element steps, one flat
-//   sequence of steps across tiles, so the pipeline never drains between
-//   tiles;
+// * a persistent workgroup per CU walks its column tiles (128 or 160
+//   output columns) and, per tile, K in 64-element steps, one flat sequence
+//   of steps across tiles, so the pipeline never drains between tiles;
 // * each step's x rows (all M) and W rows go from global memory into a slot
 //   of an LDS ring (4 to 8 slots, as many as fit) by LDS DMA
 //   (global_load_lds_dwordx4), all but one slot in flight ahead of the math:
 //   W is read from HBM exactly once, x once per tile from L2;
-// * up to 80 rows each wave multiplies its two W tiles by all M / 16 x tiles
-//   (v_mfma_f32_16x16x32_bf16, A = W, B = x^T): a W fragment feeds MT MFMAs,
-//   an x fragment two; from 96 rows the waves split the rows in two and the
-//   columns in two (half the x tiles by four W tiles each: fewer fragment
-//   reads);
+// * the waves split the rows (in one or two groups) and the tile's columns:
+//   each multiplies its W tiles by its x tiles (v_mfma_f32_16x16x32_bf16, A =
+//   W, B = x^T);
 // * an output element's whole K sum stays in one wave, in k order, so the
 //   result does not depend on the grid;
 // * the logits are bf16(acc), one rounding (lm_head has no bias); the argmax
@@ -46,23 +43,32 @@
 namespace nsg {
 namespace {
 
-constexpr int kWaves = 4;
-constexpr int kNT = 2;                     // 16-column W tiles per wave
-constexpr int kCols = kWaves * kNT * 16;   // output columns per workgroup tile
+// Shapes of a workgroup (waves, columns per tile, row groups of waves).
+// * The argmax form: eight waves by 128 columns up to 80 rows and below 65536
+//   columns, ten by 160 otherwise (x is read once per tile: 13 % fewer bytes
+//   per CU), two row groups and column groups of 32 columns, so that a SIMD
+//   holds two or three waves.  Plain greedy call at 160 rows, us: four waves
+//   by 128 columns 67.2, eight 65.4, ten 63.6; 61.4 / 59.9 / 58.2 at 128 rows;
+//   at 32 ten waves are behind (folded call 52.5 against 51.3).  (From 65536
+//   columns a key per row and column group stays within 4 * ceil(N / 128).)
+// * The logits form: four waves by 128 columns; its stores set the pace, and
+//   with more waves a whole verify forward was 4 us slower (456 against 452).
+constexpr int kTenWaveMinN = 65536;
 constexpr int kRowBytes = kHeadStep * 2;   // one row's bytes per step
 constexpr int kLdsMax = 160 * 1024;
 constexpr int kHeadMaxParts = 64;  // folded norm: partial sums per row
 constexpr int kMaxStages = 8;
 
-template <int MT>
+template <int MT, int COLS>
 constexpr int stage_bytes() {
-  return (MT * 16 + kWaves * kNT * 16) * kRowBytes;
+  return (MT * 16 + COLS) * kRowBytes;
 }
 // Ring depth: as many slots as the CU's LDS holds (4 at 160 rows, 6 at 64);
 // all but one are in flight ahead of the math.
-template <int MT>
+template <int MT, int COLS>
 constexpr int ring_stages() {
-  return kLdsMax / stage_bytes<MT>() < kMaxStages ? kLdsMax / stage_bytes<MT>() : kMaxStages;
+  return kLdsMax / stage_bytes<MT, COLS>() < kMaxStages ? kLdsMax / stage_bytes<MT, COLS>()
+                                                         : kMaxStages;
 }
 
 // One LDS DMA copy of 16 bytes per lane: lane l's 16 bytes land at LDS
@@ -88,13 +94,8 @@ __device__ __forceinline__ void dma16_nt(uint32_t lds, const void* src) {
 
 __device__ __forceinline__ uint64_t key_max(uint64_t a, uint64_t b) { return a > b ? a : b; }
 
-// Row groups of waves in the lm_head kernel: 2 from 96 rows (MT 6), else 1.
-template <int MT>
-constexpr int lm_row_split() {
-  return MT >= 6 ? 2 : 1;
-}
 
-template <int MT, bool ARG, bool FOLD>
+template <int MT, int kWaves, int kCols, int RS, bool ARG, bool FOLD>
 __global__ __launch_bounds__(kWaves * 64) void lm_head_kernel(HeadParams p) {
   static_assert(MT % 2 == 0 && MT >= 2 && MT <= kHeadMaxRows / 16, "whole x copies");
   // x: MT * 16 rows x 8 segments = 2 MT copies per step, kX per wave (the
@@ -102,18 +103,15 @@ __global__ __launch_bounds__(kWaves * 64) void lm_head_kernel(HeadParams p) {
   // same place)
   constexpr int kXAll = 2 * MT;
   constexpr int kX = (kXAll + kWaves - 1) / kWaves;
-  constexpr int kW = 2 * kNT;      // W copies per wave and step (its 32 rows x 8 segments)
+  constexpr int kW = kCols / kWaves * kRowBytes / 1024;  // W copies per wave and step
   constexpr int NI = kX + kW;      // vector-memory instructions per wave and step
-  // MFMA work of a step: RS row groups x kWaves / RS column groups of waves,
-  // each wave XT x tiles by WT W tiles (from 96 rows two row groups: each
-  // wave reads half of x's fragments and twice the W fragments, 9 instead of
-  // 12 fragment reads per 32-k at 160 rows)
-  constexpr int RS = lm_row_split<MT>();
+  // MFMA work of a step: RS row groups x CG column groups of waves, each XT x
+  // tiles by WT W tiles
   constexpr int XT = MT / RS;
-  constexpr int WT = kNT * RS;
   constexpr int CG = kWaves / RS;
-  constexpr int SB = stage_bytes<MT>();
-  constexpr int kStages = ring_stages<MT>();
+  constexpr int WT = kCols / 16 / CG;
+  constexpr int SB = stage_bytes<MT, kCols>();
+  constexpr int kStages = ring_stages<MT, kCols>();
   static_assert(kStages >= 3 && (kStages - 2) * NI <= 63, "vmcnt counts to 63");
   __shared__ __attribute__((aligned(1024))) uint8_t ring[kStages * SB];
 
@@ -151,7 +149,7 @@ __global__ __launch_bounds__(kWaves * 64) void lm_head_kernel(HeadParams p) {
   }
   const bf16* wsrc[kW];
   auto set_w = [&](int j) {  // W rows of this wave for the workgroup's tile j
-    const int c0 = ((int)blockIdx.x + j * (int)gridDim.x) * kCols + wave * kNT * 16;
+    const int c0 = ((int)blockIdx.x + j * (int)gridDim.x) * kCols + wave * (kCols / kWaves);
 #pragma unroll
     for (int i = 0; i < kW; ++i) {
       int c = c0 + wrow[i];
@@ -159,7 +157,7 @@ __global__ __launch_bounds__(kWaves * 64) void lm_head_kernel(HeadParams p) {
       wsrc[i] = p.w + (int64_t)c * p.ldw + wseg[i] * 8;
     }
   };
-  const uint32_t w_lds = ring_lds + MT * 16 * kRowBytes + wave * kNT * 16 * kRowBytes;
+  const uint32_t w_lds = ring_lds + MT * 16 * kRowBytes + wave * (kCols / kWaves) * kRowBytes;
 
   // issue cursor: steps issued so far, and the tile / step of the next one
   int issued = 0, i_tile = 0, i_step = 0, i_slot = 0;
@@ -581,31 +579,34 @@ int device_cus() {
   return cus[dev];
 }
 
+template <int MT, int NW, int COLS, int RS, bool ARG>
+int32_t launch_shape(const HeadParams& p, hipStream_t s, int* key_cols) {
+  const int tiles = (p.N + COLS - 1) / COLS;
+  const int per_cu = kLdsMax / (ring_stages<MT, COLS>() * stage_bytes<MT, COLS>());
+  const int grid = std::min(tiles, device_cus() * std::max(per_cu, 1));
+  *key_cols = NW / RS * grid;
+  if (p.sumsq)
+    hipLaunchKernelGGL((lm_head_kernel<MT, NW, COLS, RS, ARG, true>), dim3(grid), dim3(NW * 64), 0,
+                       s, p);
+  else
+    hipLaunchKernelGGL((lm_head_kernel<MT, NW, COLS, RS, ARG, false>), dim3(grid), dim3(NW * 64),
+                       0, s, p);
+  return launch_status("lm_head_kernel");
+}
+
 template <int MT>
 int32_t launch_mt(const HeadParams& p, bool argmax, hipStream_t s, int* key_cols) {
-  const int tiles = (p.N + kCols - 1) / kCols;
-  const int per_cu = kLdsMax / (ring_stages<MT>() * stage_bytes<MT>());
-  const int grid = std::min(tiles, device_cus() * std::max(per_cu, 1));
-  *key_cols = kWaves / lm_row_split<MT>() * grid;
-  const dim3 g(grid), b(kWaves * 64);
-  if (p.sumsq) {
-    if (argmax)
-      hipLaunchKernelGGL((lm_head_kernel<MT, true, true>), g, b, 0, s, p);
-    else
-      hipLaunchKernelGGL((lm_head_kernel<MT, false, true>), g, b, 0, s, p);
-  } else {
-    if (argmax)
-      hipLaunchKernelGGL((lm_head_kernel<MT, true, false>), g, b, 0, s, p);
-    else
-      hipLaunchKernelGGL((lm_head_kernel<MT, false, false>), g, b, 0, s, p);
+  if (!argmax) return launch_shape<MT, 4, 128, MT >= 6 ? 2 : 1, false>(p, s, key_cols);
+  if constexpr (MT >= 6) {
+    if (p.N >= kTenWaveMinN) return launch_shape<MT, 10, 160, 2, true>(p, s, key_cols);
   }
-  return launch_status("lm_head_kernel");
+  return launch_shape<MT, 8, 128, 2, true>(p, s, key_cols);
 }
 
 template <int MT>
 bool fold_fits_mt(int M, int parts) {
   const int64_t n16 = (int64_t)M * parts / 4;
-  return ((n16 + 63) / 64) * 1024 <= stage_bytes<MT>() - 1024;
+  return ((n16 + 63) / 64) * 1024 <= stage_bytes<MT, 128>() - 1024;  // (the smaller slot)
 }
 
 }  // namespace
