@@ -1,7 +1,8 @@
 // Verify attention for gfx950: ragged multi-query attention of the draft's
 // k tokens plus the bonus token against the NHD paged KV cache, with GQA and
 // the bottom-right causal rule.  The same kernel serves decode (q_len = 1),
-// verify (q_len = k + 1) and chunked prefill (any q_len).
+// verify (q_len = k + 1) and prefill chunks that do not fill the prefill
+// kernel (prefill_attention.hip; see prefill_rows).
 //
 // Reference semantics: nano_sglang/model/causal_lm.py:359-471 (the PyTorch
 // packed-attention fallbacks that define what the FlashInfer call at
