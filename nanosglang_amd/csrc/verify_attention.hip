@@ -797,8 +797,13 @@ int32_t launch_rt(const nsg_attn_plan_t* plan, const AttnParams& prm, const int*
 template <int D>
 int32_t launch_d(const nsg_attn_plan_t* plan, const AttnParams& prm, const int* merge,
                  hipStream_t stream) {
-  if ((plan->row_tiles == 8 || plan->row_tiles == 16) && plan->kv_groups == 1)
+  if ((plan->row_tiles == 8 || plan->row_tiles == 16) && plan->kv_groups == 1) {
+    // the prefill kernel sweeps an item's KV range from token 0 and merges nothing
+    NSG_CHECK_ARG(plan->max_splits == 1 && plan->num_merge == 0,
+                  "prefill tiles are never split: plan has %d KV splits, %d merge items",
+                  plan->max_splits, plan->num_merge);
     return launch_prefill_attn(D, plan->row_tiles / 2, plan->num_work, prm, stream);
+  }
   switch (plan->row_tiles) {
     case 1: return launch_rt<D, 1>(plan, prm, merge, stream);
     case 2: return launch_rt<D, 2>(plan, prm, merge, stream);
@@ -1027,7 +1032,12 @@ int32_t plan_impl(const int32_t* qo_indptr_h, const int32_t* kv_indptr_h,
       std::max<long long>(1, ((long long)(kMaxItemPages - 2) * page_size) / kTokIt);
   chunk_it = std::min(chunk_it, max_chunk_it);
   if (fixed_kv_len > 0) chunk_it = std::max<long long>(chunk_it, (fixed_kv_len + kTokIt - 1) / kTokIt);
-  if (prefill) chunk_it = max_chunk_it;  // never split (prefill_rows bounds the pages)
+  // Prefill tiles are never split: the longest tile's steps (not max_chunk_it,
+  // which rounds down to whole steps of pages below 32 tokens; prefill_rows
+  // bounds the pages).
+  if (prefill)
+    for (const Group& g : groups)
+      chunk_it = std::max<long long>(chunk_it, (g.kv_end + kTokIt - 1) / kTokIt);
 
   int n = 0, max_splits = 0, n_merge = 0;
   std::vector<int> split_counts(groups.size());

@@ -44,6 +44,23 @@ def test_prefill_tile_edges(Hq, Hkv, D, P, causal):
 
 
 @pytest.mark.parametrize("Hq,Hkv,D", [(14, 2, 64), (32, 8, 128)])
+def test_prefill_at_the_end_of_the_page_list(Hq, Hkv, D):
+    """Pages of one token, contexts around the 992 tokens that are whole 32-token
+    steps of the 1022 an item's page list holds: one item per tile to the end."""
+    kv = [992, 993, 1010, 1022]
+    c = workloads.verify_attention_batch(batch=4, kv_lens=kv, q_lens=kv, page_size=1,
+                                         num_qo_heads=Hq, num_kv_heads=Hkv, head_dim=D,
+                                         num_pages=sum(kv) + 3, seed=D)
+    print(f"case: {Hq}/{Hkv} x {D}, pages of 1, contexts {kv}", flush=True)
+    got, w = _run(c, Hq, Hkv, D, True)
+    assert w.plan_info.max_splits == 1
+    ref = verify_attention(c["q"], c["k"], c["v"], c["qo_indptr"], c["kv_indptr"],
+                           c["kv_indices"], c["kv_last_page_len"], c["sm_scale"], True)
+    assert w.check_flags() == 0
+    assert (np.abs(got - ref) <= 2e-3 + 2.0 ** -8 * np.abs(ref)).all()
+
+
+@pytest.mark.parametrize("Hq,Hkv,D", [(14, 2, 64), (32, 8, 128)])
 def test_prefill_growing_scores_and_bad_page(Hq, Hkv, D):
     """Scores that grow along the context rescale the running sums often; a page
     id outside the pool raises the flag and leaves other requests alone."""

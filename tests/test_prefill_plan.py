@@ -61,3 +61,39 @@ def test_which_batches_get_prefill_tiles(q, kv, heads, prefill):
     assert (pl.row_tiles >= 8) == prefill
     if not prefill:      # the verify kernel's forms are what they were
         assert pl.row_tiles <= 4 and pl.q_tile_tokens * (heads[0] // heads[1]) <= 64
+
+
+@pytest.mark.parametrize("P", [1, 2, 4, 8, 16, 32])
+@pytest.mark.parametrize("Hq,Hkv,D", [(14, 2, 64), (32, 8, 128)])
+def test_items_are_never_split_up_to_the_page_list(Hq, Hkv, D, P):
+    """The prefill kernel sweeps an item's whole KV range and merges nothing, so
+    every query tile is one item up to the 1022 pages an item's list holds (also
+    where 1022 pages are no whole number of 32-token steps); past them the batch
+    is the verify kernel's."""
+    full = 1022 * P
+    for L in (full, full - 1, full // 32 * 32, min(full, full // 32 * 32 + 1)):
+        B = max(2, 16384 // L)
+        pl, work, qo, kvp = _plan([L] * B, [L] * B, Hq, Hkv, D, P=P)
+        T = pl.q_tile_tokens
+        assert pl.row_tiles >= 8 and pl.max_splits == 1 and pl.num_merge == 0, (P, L)
+        assert len(work) == B * -(-L // T), (P, L)
+        assert sorted(zip(work[:, 0], work[:, 1], work[:, 4], work[:, 5])) == [
+            (b * L + q, min(T, L - q), 0, min(q + T, L)) for b in range(B) for q in range(0, L, T)]
+    pl, _, _, _ = _plan([full + 1] * 16, [full + 1] * 16, Hq, Hkv, D, P=P)
+    assert pl.row_tiles <= 4
+
+
+def test_a_prefill_plan_with_splits_is_refused():
+    """A record that claims prefill tiles and KV splits is no plan of this
+    library: nsg_attn_run answers with an error and launches nothing (the pointers
+    here are never followed)."""
+    pl, _, _, _ = _plan([300] * 4, [300] * 4, 14, 2, 64)
+    assert pl.row_tiles == 8
+    lib = _native.load()
+    dummy = C.create_string_buffer(256)
+    ptr = [C.cast(dummy, C.c_void_p)] * 9
+    for field, value in (("max_splits", 2), ("num_merge", 1)):
+        bad = AttnPlan.from_buffer_copy(pl)
+        setattr(bad, field, value)
+        rc = lib.nsg_attn_run(C.byref(bad), *ptr, 16, 100, 0.125, 1, ptr[0], 256, None)
+        assert rc != 0 and b"prefill" in lib.nsg_last_error() and b"split" in lib.nsg_last_error()
