@@ -1096,6 +1096,7 @@ int32_t plan_impl(const int32_t* qo_indptr_h, const int32_t* kv_indptr_h,
     for (size_t gi = 0; gi < groups.size(); ++gi)
       order[(size_t)at[(size_t)(most - steps(groups[gi]))]++] = (int)gi;
   }
+  const bool all_at_once = (long long)n * num_kv_heads <= num_cus;
   n = 0;
   int m = 0;
   for (size_t oi = 0; oi < groups.size(); ++oi) {
@@ -1113,18 +1114,28 @@ int32_t plan_impl(const int32_t* qo_indptr_h, const int32_t* kv_indptr_h,
       w[4] = w[5] = w[6] = w[7] = 0;
       ++m;
     }
-    // even shares of the group's steps (each at most chunk_it): with whole
-    // chunks and a short rest the last wave of workgroups ends unevenly
-    // (large shape, three draws of lengths: 308 / 302 / 298 -> 299 / 294 / 292 us)
+    // The tile's steps in even shares (each at most chunk_it), or in whole
+    // chunks and a rest.  One KV group (many workgroups per CU): even shares,
+    // for a short rest lets the last workgroups end unevenly (large shape,
+    // three draws of lengths: 308 / 302 / 298 -> 299 / 294 / 292 us).  Several
+    // KV groups (one workgroup per CU): even shares when every workgroup runs
+    // at once (level with chunks), and past that for two splits (48 rows over
+    // 4000, 64 / 8 heads of 128: 92 in chunks, 66 in shares) or a rest of at
+    // most an eighth (128 over 4000, 16 / 2 heads: 63, 47); else whole chunks,
+    // whose rests free CUs early for the second round (48 over 1200, 32 / 32
+    // heads, 288 workgroups: 15.4 in chunks, 22.3 in shares).
     const long long its = (g.kv_end + kTokIt - 1) / kTokIt;
+    const long long rest = its - (ns - 1) * chunk_it;
+    const bool even = KS == 1 || all_at_once || ns == 2 || 8 * rest <= chunk_it;
+    auto cut = [&](int s) { return (even ? its * s / ns : s * chunk_it) * kTokIt; };
     for (int s = 0; s < ns; ++s) {
       int32_t* w = work_h + (size_t)n * NSG_ATTN_WORK_INTS;
       w[0] = qs;
       w[1] = g.qn;
       w[2] = g.lim0;
       w[3] = kv_indptr_h[g.b];
-      w[4] = (int)(its * s / ns * kTokIt);
-      w[5] = (int)std::min<long long>(g.kv_end, its * (s + 1) / ns * kTokIt);
+      w[4] = (int)cut(s);
+      w[5] = (int)std::min<long long>(g.kv_end, cut(s + 1));
       w[6] = ns;
       w[7] = 0;
       ++n;
