@@ -2,7 +2,7 @@
 // k tokens plus the bonus token against the NHD paged KV cache, with GQA and
 // the bottom-right causal rule.  The same kernel serves decode (q_len = 1),
 // verify (q_len = k + 1) and prefill chunks that do not fill the prefill
-// kernel (prefill_attention.hip; see prefill_rows).
+// kernel (prefill_attention.hip; see prefill_shape).
 //
 // Reference semantics: nano_sglang/model/causal_lm.py:359-471 (the PyTorch
 // packed-attention fallbacks that define what the FlashInfer call at
@@ -31,6 +31,7 @@
 //     from the LDS tile in the same token order;
 //   - the prefetched registers go to the other LDS buffer; one barrier.
 #include <algorithm>
+#include <cmath>
 #include <numeric>
 #include <type_traits>
 #include <cstdarg>
@@ -875,26 +876,32 @@ void fixed_capacity(int batch, int max_ql, int G, int num_kv_heads, int num_cus,
   *max_merge = groups;
 }
 
-// Rows per workgroup of the prefill kernel (prefill_attention.hip) for this
-// batch, or 0 for the verify kernel.  It does not split the KV range, so it
-// is taken when its tiles are well filled (a 256-row workgroup at least half,
-// a 128-row one three quarters) and there are enough of them: one workgroup
-// per CU, or a third of that with contexts of at most 2048 tokens.  Measured
-// (us, verify kernel -> this one): a batch of 32 prompts of 100 - 512 tokens,
-// 14 / 2 heads of 64, 42.5 -> 23.4; two prompts of 2048 - 8192, 32 / 8 heads
-// of 128, 1081 -> 609; 16 x 32 query tokens over 100 - 640, 40 -> 23.  Below
-// the line the verify kernel's KV groups and splits are ahead: one prompt of
-// 300 tokens (34 workgroups) 8.0 against 10.0, 2 x 512 tokens over 4000 -
-// 8000 (116 long workgroups) 66 against 101.
-// 256 rows only at head dim 128, where two wave groups then alternate
-// (prefill_attention.hip); at 64 the shorter 128-row workgroups were ahead
-// throughout (23.4 against 27.9 us on the 32 prompts).
-int prefill_rows(const int32_t* qo, const int32_t* kvp, int batch, int G, int num_kv_heads,
-                 int head_dim, int page_size, int num_cus) {
+// The prefill kernel's (prefill_attention.hip) shape for a batch.
+struct PrefillShape {
+  int rows = 0;         // per workgroup, 128 or 256; 0: the verify kernel
+  long long wgs = 0;    // workgroups
+};
+
+// The prefill kernel does not split the KV range, so it is considered when its
+// tiles are well filled (a 256-row workgroup at least half, a 128-row one three
+// quarters) and there are enough of them: one workgroup per CU, or a third of
+// that with contexts of at most 2048 tokens.  256 rows only at head dim 128,
+// where two wave groups then alternate; at 64 the shorter 128-row workgroups
+// were ahead throughout (23.4 against 27.9 us on 32 prompts of 100 - 512
+// tokens); and not for four or more rounds of contexts up to 384 tokens, whose
+// few steps do not pay for the longer start (64 prompts of 128, 32 / 8 heads:
+// 256 rows 74 us, 128 rows 52, verify kernel 56).  From two workgroups per CU on
+// it is ahead; below, prefill_ahead decides.  Over 4,127 batches of nine head
+// shapes 1,913 take the prefill kernel, at 0.57 of the verify kernel's time
+// (geometric mean); six are slower by more than 3 %, the slowest 1.12 (64
+// prompts of 128, 32 / 32 heads of 128: 60.6 -> 67.8).
+PrefillShape prefill_shape(const int32_t* qo, const int32_t* kvp, int batch, int G,
+                           int num_kv_heads, int head_dim, int page_size, int num_cus) {
   int max_pages = 0;
   for (int b = 0; b < batch; ++b)
     if (qo[b + 1] > qo[b]) max_pages = std::max(max_pages, kvp[b + 1] - kvp[b]);
-  if (max_pages > kMaxItemPages - 2) return 0;  // the item's page list
+  if (max_pages > kMaxItemPages - 2) return {};  // the item's page list
+  const long long ctx = (long long)max_pages * page_size;
   for (int rows : {256, 128}) {
     if (rows == 256 && head_dim == 64) continue;
     const int T = rows / G;
@@ -905,11 +912,48 @@ int prefill_rows(const int32_t* qo, const int32_t* kvp, int batch, int G, int nu
       used += (long long)ql * G;
     }
     const long long wgs = tiles * num_kv_heads;
-    const bool fills = wgs >= num_cus ||
-                       (3 * wgs >= num_cus && (long long)max_pages * page_size <= 2048);
-    if (4 * used >= (rows == 256 ? 2 : 3) * tiles * rows && fills) return rows;
+    if (rows == 256 && ctx <= 384 && wgs >= 4ll * num_cus) continue;
+    const bool fills = wgs >= num_cus || (3 * wgs >= num_cus && ctx <= 2048);
+    if (4 * used >= (rows == 256 ? 2 : 3) * tiles * rows && fills) return {rows, wgs};
   }
-  return 0;
+  return {};
+}
+
+// Below two workgroups per CU the verify kernel's KV groups and splits can be
+// ahead, so both kernels' times are estimated (us, fitted to 3,890 batches of
+// nine head shapes, page size 16, each run on both: within 6 - 13 % rms).
+// Prefill: the start and the longest tile's 64-token steps, or all steps and
+// workgroups over the CUs.  Verify: with several KV groups the longest item's
+// 32-token steps per group and round, with one all steps over the CUs (or the
+// longest item), and the merge launch.  The prefill kernel is taken when its
+// estimate is 10 % shorter (20 % for groups above 16, where the verify kernel's
+// tiles are as tall in both regimes).  Without the comparison 86 of the batches
+// were 3 - 77 % slower than on the verify kernel (16 x 16 query tokens over 600,
+// 64 / 1 heads of 128: 15.7 -> 27.8; 256 over 2040, 40 / 8: 51 -> 70).
+bool prefill_ahead(const PrefillShape& pre, int head_dim, int G, int num_cus, long long steps,
+                   long long longest, int kv_groups, int row_tiles, long long items,
+                   long long item_steps, long long longest_item, bool split) {
+  struct Fit { double start, step, fill, all_steps, wg; int slots; };
+  const Fit f = head_dim == 64   ? Fit{4.6, 0.98, 3.3, 0.75, 1.43, 3}
+                : pre.rows == 128 ? Fit{5.5, 2.0, 5.5, 1.46, 3.45, 2}
+                                  : Fit{7.4, 1.75, 5.4, 2.12, 6.8, 1};
+  const double cus = num_cus;
+  const double prefill_us =
+      f.start + std::max(f.step * longest + f.fill * std::min(1.0, pre.wgs / (f.slots * cus)),
+                         (f.all_steps * steps + f.wg * pre.wgs) / cus);
+  double verify_us;
+  if (kv_groups > 1) {
+    const double rounds = std::ceil(items / cus);
+    const double sweep =
+        std::max(longest_item * rounds, item_steps / cus) / kv_groups * (row_tiles > 1 ? 1.56 : 1.0);
+    verify_us = head_dim == 64 ? 2.2 + 0.53 * sweep + 2.06 * rounds + (split ? 2.2 : 0.0)
+                               : 2.6 + 0.78 * sweep + 2.5 * rounds + (split ? 1.9 : 0.0);
+  } else {
+    const double sweep = std::max((double)longest_item, item_steps / cus);
+    verify_us = head_dim == 64 ? 19.6 + 0.289 * sweep + (split ? 7.4 : 0.0)
+                               : 29.3 + 0.516 * sweep + (split ? 10.8 : 0.0);
+  }
+  return prefill_us <= (G > 16 ? 0.8 : 0.9) * verify_us;
 }
 
 int max_splits_planned(const std::vector<int>& split_counts) {
@@ -1000,20 +1044,18 @@ int32_t plan_impl(const int32_t* qo_indptr_h, const int32_t* kv_indptr_h,
   // kMinSplitSteps steps per group: its partial rows cost about as much
   // traffic as one step of K and V.
   const long long t1 = target_items(1, num_cus, num_kv_heads);
-  bool latency;
-  int T;
-  const int prefill = fixed_work >= 0 ? 0
-                      : prefill_rows(qo_indptr_h, kv_indptr_h, batch, G, num_kv_heads, head_dim,
-                                     page_size, num_cus);
-  if (prefill) {
-    latency = false;
-    T = prefill / G;
-    if (int32_t rc = make_groups(T)) return rc;
-  } else if (fixed_work >= 0) {
+  bool latency = false;
+  int T = 0;
+  PrefillShape pre;
+  if (fixed_work < 0)
+    pre = prefill_shape(qo_indptr_h, kv_indptr_h, batch, G, num_kv_heads, head_dim, page_size,
+                        num_cus);
+  const bool compare = pre.rows && pre.wgs < 2ll * num_cus;
+  if (fixed_work >= 0) {
     latency = page_size >= kMinGroupPage && fixed_kv_len > 0;
     T = q_tile_tokens(G, max_ql, latency);
     if (int32_t rc = make_groups(T)) return rc;
-  } else {
+  } else if (!pre.rows || compare) {
     T = q_tile_tokens(G, max_ql, false);
     if (int32_t rc = make_groups(T)) return rc;
     latency = page_size >= kMinGroupPage && (total_it + t1 - 1) / t1 <= kMinSplitSteps;
@@ -1022,19 +1064,55 @@ int32_t plan_impl(const int32_t* qo_indptr_h, const int32_t* kv_indptr_h,
       if (int32_t rc = make_groups(T)) return rc;
     }
   }
+  // KV groups and the steps of an item; a work item's page ids must fit the
+  // kernel's LDS list (kMaxItemPages)
+  int KS = 1;
+  long long chunk_it = 0;
+  auto set_chunk = [&]() {
+    KS = latency ? kv_groups_max(head_dim) : 1;
+    const long long tgt = target_items(KS, num_cus, num_kv_heads);
+    chunk_it = std::max<long long>((long long)(KS > 1 ? kMinGroupSteps : kMinSplitSteps) * KS,
+                                   (total_it + tgt - 1) / tgt);
+    const long long max_chunk_it =
+        std::max<long long>(1, ((long long)(kMaxItemPages - 2) * page_size) / kTokIt);
+    chunk_it = std::min(chunk_it, max_chunk_it);
+    if (fixed_kv_len > 0)
+      chunk_it = std::max<long long>(chunk_it, (fixed_kv_len + kTokIt - 1) / kTokIt);
+  };
+  if (compare) {
+    set_chunk();
+    long long items = 0, longest_item = 0, steps = 0, longest = 0;
+    for (const Group& g : groups) {
+      const long long its = (g.kv_end + kTokIt - 1) / kTokIt;
+      items += (its + chunk_it - 1) / chunk_it;
+      longest_item = std::max(longest_item, std::min(its, chunk_it));
+    }
+    const bool split = items > (long long)groups.size();
+    const long long item_steps = total_it;
+    const int rt = (T * G + 15) / 16;
+    if (int32_t rc = make_groups(pre.rows / G)) return rc;
+    for (const Group& g : groups) {
+      steps += (g.kv_end + 63) / 64;
+      longest = std::max<long long>(longest, (g.kv_end + 63) / 64);
+    }
+    if (!prefill_ahead(pre, head_dim, G, num_cus, steps * num_kv_heads, longest, KS, rt,
+                       items * num_kv_heads, item_steps * num_kv_heads, longest_item, split)) {
+      pre.rows = 0;
+      if (int32_t rc = make_groups(T)) return rc;
+    }
+  }
+  const int prefill = pre.rows;
+  if (prefill) {
+    latency = false;
+    T = prefill / G;
+    if (!compare)
+      if (int32_t rc = make_groups(T)) return rc;
+  }
   const int RT = prefill ? prefill / 16 : (T * G + 15) / 16;
-  const int KS = latency ? kv_groups_max(head_dim) : 1;
-  const long long tgt = target_items(KS, num_cus, num_kv_heads);
-  long long chunk_it = std::max<long long>(
-      (long long)(KS > 1 ? kMinGroupSteps : kMinSplitSteps) * KS, (total_it + tgt - 1) / tgt);
-  // a work item's page ids must fit the kernel's LDS list (kMaxItemPages)
-  const long long max_chunk_it =
-      std::max<long long>(1, ((long long)(kMaxItemPages - 2) * page_size) / kTokIt);
-  chunk_it = std::min(chunk_it, max_chunk_it);
-  if (fixed_kv_len > 0) chunk_it = std::max<long long>(chunk_it, (fixed_kv_len + kTokIt - 1) / kTokIt);
-  // Prefill tiles are never split: the longest tile's steps (not max_chunk_it,
-  // which rounds down to whole steps of pages below 32 tokens; prefill_rows
-  // bounds the pages).
+  set_chunk();
+  // Prefill tiles are never split: the longest tile's steps (not the capped
+  // chunk, which rounds down to whole steps of pages below 32 tokens;
+  // prefill_shape bounds the pages).
   if (prefill)
     for (const Group& g : groups)
       chunk_it = std::max<long long>(chunk_it, (g.kv_end + kTokIt - 1) / kTokIt);

@@ -97,3 +97,27 @@ def test_a_prefill_plan_with_splits_is_refused():
         setattr(bad, field, value)
         rc = lib.nsg_attn_run(C.byref(bad), *ptr, 16, 100, 0.125, 1, ptr[0], 256, None)
         assert rc != 0 and b"prefill" in lib.nsg_last_error() and b"split" in lib.nsg_last_error()
+
+
+@pytest.mark.parametrize("q,kv,heads,row_tiles", [
+    # fewer than two workgroups per CU, measured ahead on the verify kernel
+    ([16] * 16, [600] * 16, (64, 1, 128), 0),
+    ([256], [300], (64, 1, 128), 0),
+    ([256], [2040], (40, 8, 128), 0),
+    ([1024], [2040], (16, 2, 128), 0),
+    ([1024], [1200], (12, 12, 64), 0),
+    # ... and on the prefill kernel
+    ([1000], [1000], (32, 8, 128), 16),
+    ([500], [500], (32, 8, 128), 8),
+    ([48] * 16, [1200] * 16, (32, 8, 128), 16),
+    ([512] * 2, [512] * 2, (14, 2, 64), 8),
+    # many rounds of short contexts: 128 rows
+    ([128] * 64, [128] * 64, (32, 8, 128), 8),
+    ([256] * 16, [256] * 16, (64, 8, 128), 8),
+    ([512] * 32, [512] * 32, (32, 8, 128), 16),
+])
+def test_which_kernel_a_batch_gets(q, kv, heads, row_tiles):
+    """Row tiles of the prefill kernel (0: the verify kernel's 1 .. 4), as measured
+    on both."""
+    pl, _, _, _ = _plan(q, kv, *heads)
+    assert pl.row_tiles == row_tiles if row_tiles else pl.row_tiles <= 4
