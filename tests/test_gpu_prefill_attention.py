@@ -13,13 +13,14 @@ from oracle.verify_attention import verify_attention
 pytestmark = pytest.mark.gpu
 
 
-def _run(c, Hq, Hkv, D, causal):
+def _run(c, Hq, Hkv, D, causal, row_tiles=None):
     dev = lambda x: torch.from_numpy(np.ascontiguousarray(x)).cuda().bfloat16()  # noqa: E731
     w = BatchPrefillWithPagedKVCacheWrapper(
         torch.empty(1 << 20, dtype=torch.uint8, device="cuda"), "NHD", num_cus=8)
     w.plan(c["qo_indptr"], c["kv_indptr"], c["kv_indices"], c["kv_last_page_len"], Hq, Hkv, D,
            c["page_size"], causal=causal)
     assert w.plan_info.row_tiles >= 8, "not the prefill kernel"
+    assert row_tiles in (None, w.plan_info.row_tiles)
     out = w.run(dev(c["q"]), (dev(c["k"]), dev(c["v"])))
     return out.float().cpu().numpy(), w
 
@@ -36,7 +37,30 @@ def test_prefill_tile_edges(Hq, Hkv, D, P, causal):
                                          num_qo_heads=Hq, num_kv_heads=Hkv, head_dim=D,
                                          num_pages=sum(-(-L // P) for L in kv) + 3, seed=D + P)
     print(f"case: {Hq}/{Hkv} x {D}, pages of {P}, causal {causal}", flush=True)
-    got, w = _run(c, Hq, Hkv, D, causal)
+    got, w = _run(c, Hq, Hkv, D, causal, row_tiles=8 if D == 64 else 16)
+    ref = verify_attention(c["q"], c["k"], c["v"], c["qo_indptr"], c["kv_indptr"],
+                           c["kv_indices"], c["kv_last_page_len"], c["sm_scale"], causal)
+    assert w.check_flags() == 0
+    assert (np.abs(got - ref) <= 2e-3 + 2.0 ** -8 * np.abs(ref)).all()
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("Hq,Hkv,P,ql", [
+    (32, 8, 16, [30, 31, 32, 25, 30, 32, 28, 31, 32, 30, 29]),      # chunks over a cached prefix
+    (4, 4, 1, [127, 100, 120, 128, 126, 97, 125, 128, 119, 128, 120]),
+    (64, 8, 128, [15, 16, 14, 12, 16, 15, 16, 13, 16, 15, 16]),
+    (16, 2, 4, None)])                                              # short prompts, many rounds
+def test_128_row_tiles_at_head_dim_128(Hq, Hkv, P, ql, causal):
+    """The two-slot ring of 128 rows at head dim 128: contexts around one, two and
+    three of its 64-token steps and long ones."""
+    kv = [63, 64, 65, 127, 128, 129, 193, 257, 320, 349, 384]
+    ql, kv = (kv, kv) if ql is None else (
+        [min(q, L) for q, L in zip(ql, kv)] + ql[:2], kv + [1000, 1009])
+    c = workloads.verify_attention_batch(batch=len(kv), kv_lens=kv, q_lens=ql, page_size=P,
+                                         num_qo_heads=Hq, num_kv_heads=Hkv, head_dim=128,
+                                         num_pages=sum(-(-L // P) for L in kv) + 3, seed=P)
+    print(f"case: {Hq}/{Hkv} x 128, pages of {P}, causal {causal}", flush=True)
+    got, w = _run(c, Hq, Hkv, 128, causal, row_tiles=8)
     ref = verify_attention(c["q"], c["k"], c["v"], c["qo_indptr"], c["kv_indptr"],
                            c["kv_indices"], c["kv_last_page_len"], c["sm_scale"], causal)
     assert w.check_flags() == 0
