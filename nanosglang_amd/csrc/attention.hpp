@@ -89,7 +89,7 @@ __device__ __forceinline__ int swz_v(int t) {
 
 
 // The prefill kernel (prefill_attention.hip): unsplit work items of up to
-// 32 * waves query rows, waves = 4 or 8.
+// 32 * waves query rows, waves = 4, or 8 at head dim 128.
 int32_t launch_prefill_attn(int head_dim, int waves, int num_work, const AttnParams& prm,
                             hipStream_t stream);
 

@@ -69,7 +69,7 @@ constexpr int prefill_ring() {
 }
 
 template <int D, int NW>
-__global__ __launch_bounds__(NW * 64, D == 64 && NW == 4 ? 3 : 2) void prefill_attn_kernel(AttnParams p) {
+__global__ __launch_bounds__(NW * 64, D == 64 ? 3 : 2) void prefill_attn_kernel(AttnParams p) {
   constexpr int KC = D / 16;              // k chunks of S^T = K Q^T
   constexpr int DT = D / 32;              // d tiles of O^T
   constexpr int CPR = D / 8;              // 16-byte chunks per token row
@@ -78,7 +78,7 @@ __global__ __launch_bounds__(NW * 64, D == 64 && NW == 4 ? 3 : 2) void prefill_a
   constexpr int NR = kStep / TPI / NW;    // row blocks a wave copies per step (K and V each)
   constexpr int NI = 2 * NR;              // copies per wave per step
   constexpr int kNBuf = prefill_ring<D, NW>();
-  constexpr bool PP = NW == 8 && D == 128;  // two wave groups half a step apart
+  constexpr bool PP = NW == 8;              // (head dim 128 only) two wave groups half a step apart
   static_assert(NR >= 1 && (kNBuf - 1) * NI <= 63, "vmcnt counts to 63");
   __shared__ __attribute__((aligned(1024))) bf16 ring[kNBuf][2][TILE];
   __shared__ int s_pages[kMaxItemPages];
@@ -363,8 +363,6 @@ int32_t launch_prefill_attn(int head_dim, int waves, int num_work, const AttnPar
   const dim3 grid(prm.Hkv, num_work), block(waves * 64);
   if (head_dim == 64 && waves == 4)
     hipLaunchKernelGGL((prefill_attn_kernel<64, 4>), grid, block, 0, stream, prm);
-  else if (head_dim == 64 && waves == 8)
-    hipLaunchKernelGGL((prefill_attn_kernel<64, 8>), grid, block, 0, stream, prm);
   else if (head_dim == 128 && waves == 4)
     hipLaunchKernelGGL((prefill_attn_kernel<128, 4>), grid, block, 0, stream, prm);
   else if (head_dim == 128 && waves == 8)
