@@ -434,18 +434,23 @@ int32_t nsg_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, const
  * several tensors stacked -- q/k/v, gate/up -- keep their own scales).  Each
  * weight is dequantised to bf16(float(w8) * w_scale[row]), the arithmetic of
  * FP8Linear.forward's w8.to(bf16) * scale (:49-52), and the product then runs
- * exactly as nsg_linear / nsg_linear_rope_kv on those bf16 weights (bf16 MFMA,
- * fp32 accumulation), streaming half the weight bytes.  SwiGLU: w8 and
- * w_scale have 2N rows.  Other arguments as in the bf16 entry points. */
+ * as nsg_linear / nsg_linear_rope_kv on those bf16 weights (bf16 MFMA, fp32
+ * accumulation), streaming half the weight bytes; bit for bit, except that the
+ * fp32 sums may run in another order for SwiGLU above 32 rows and, for SwiGLU
+ * of large weights and the *_ws form below, with FP8 rows that are not 16-byte
+ * aligned.  SwiGLU: w8 and w_scale have 2N rows.  Other arguments as in the
+ * bf16 entry points. */
 int32_t nsg_linear_fp8(const void* x, int64_t ldx, const void* w8, int64_t ldw8,
                        const float* w_scale, const void* bias, void* y, int64_t ldy, int32_t M,
                        int32_t N, int32_t K, int32_t epilogue, nsg_stream_t stream);
 
-/* The same two with device memory for fp32 partial sums, so that large weights
- * with few output columns can split K over the GPU.  nsg_linear_workspace_bytes:
- * the bytes (16-byte aligned, no initial contents needed) that such a split
- * takes at this shape; 0: none is made.  With less or no workspace they are
- * nsg_linear / nsg_linear_fp8.  Calls that share a workspace must not overlap. */
+/* The same two for callers that can give device memory for fp32 partial sums:
+ * large weights may run on another kernel (other order of the fp32 sums), with
+ * K split over the GPU where the output columns are few.
+ * nsg_linear_workspace_bytes: the bytes (16-byte aligned, no initial contents
+ * needed) that such a split takes at this shape; 0: K is not split and no
+ * workspace is touched.  With less than that they are nsg_linear /
+ * nsg_linear_fp8.  Calls that share a workspace must not overlap. */
 int64_t nsg_linear_workspace_bytes(int32_t M, int32_t N, int32_t K, int32_t epilogue);
 int32_t nsg_linear_ws(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias,
                       void* y, int64_t ldy, int32_t M, int32_t N, int32_t K, int32_t epilogue,

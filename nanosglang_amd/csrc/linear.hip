@@ -804,12 +804,16 @@ static bool ring_swiglu_big(int M, int N, int K) {
          (tiles >= 154 || (tiles >= 128 && M > 32));
 }
 
+static bool ring_bias_big(int M, int N, int K) {
+  return M >= kRingBiasMinRows && N < kWideN && (int64_t)N * K >= kRingBiasWeight &&
+         ring_linear_fits(M, N, K);
+}
+
 extern "C" int64_t nsg_linear_workspace_bytes(int32_t M, int32_t N, int32_t K,
                                               int32_t epilogue) {
-  if (epilogue != NSG_LINEAR_BIAS || M < kRingBiasMinRows || N >= kWideN ||
-      (int64_t)N * K < kRingBiasWeight || !ring_linear_fits(M, N, K))
-    return 0;
-  return (int64_t)ring_linear_splits(N, K) * M * N * (int64_t)sizeof(float);
+  if (epilogue != NSG_LINEAR_BIAS || N < 1 || K < 1 || !ring_bias_big(M, N, K)) return 0;
+  const int splits = ring_linear_splits(N, K);
+  return splits > 1 ? (int64_t)splits * M * N * (int64_t)sizeof(float) : 0;
 }
 
 extern "C" int32_t nsg_linear_max_rows(void) { return kMaxMT * 16; }
@@ -881,7 +885,7 @@ bool head_route(const LinParams& p) {
 int32_t linear_impl(const void* x, int64_t ldx, const void* w, const void* w8, int64_t ldw,
                     const float* w_scale, const void* bias, void* y, int64_t ldy, int32_t M,
                     int32_t N, int32_t K, int32_t epilogue, nsg_stream_t stream,
-                    const NormFold* nf = nullptr, void* workspace = nullptr,
+                    const NormFold* nf = nullptr, bool ws_form = false, void* workspace = nullptr,
                     int64_t workspace_bytes = 0) {
   NSG_CHECK_ARG(M >= 0 && N > 0 && K > 0, "M %d, N %d, K %d", M, N, K);
   if (M == 0) {
@@ -924,10 +928,14 @@ int32_t linear_impl(const void* x, int64_t ldx, const void* w, const void* w8, i
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool silu = epilogue == NSG_LINEAR_SILU_MUL;
   const int64_t ring_ws = nsg_linear_workspace_bytes(M, N, K, epilogue);
+  // (the ring's copies take 16-byte aligned FP8 rows; the bias form is the
+  // *_ws entry points' only, so that nsg_linear stays nsg_linear_rope_kv's
+  // projection bit for bit)
   if (!p.sumsq_in && !p.residual && (w || (ldw % 16 == 0 && (uintptr_t)w8 % 16 == 0)) &&
       (silu ? ring_swiglu_big(M, N, K)
-            : ring_ws > 0 && workspace && workspace_bytes >= ring_ws &&
-                  (uintptr_t)workspace % 16 == 0)) {
+            : ws_form && ring_bias_big(M, N, K) &&
+                  (ring_ws == 0 || (workspace && workspace_bytes >= ring_ws &&
+                                    (uintptr_t)workspace % 16 == 0)))) {
     const RingLinearParams rp{p.x, w ? w : w8, p.w_scale, p.bias, p.y,
                               static_cast<float*>(workspace), ldx, ldw, ldy, M, N, K,
                               silu ? 1 : ring_linear_splits(N, K)};
@@ -1034,7 +1042,7 @@ extern "C" int32_t nsg_linear_ws(const void* x, int64_t ldx, const void* w, int6
                                  int64_t workspace_bytes, nsg_stream_t stream) {
   NSG_CHECK_ARG(w, "null weight");
   return linear_impl(x, ldx, w, nullptr, ldw, nullptr, bias, y, ldy, M, N, K, epilogue, stream,
-                     nullptr, workspace, workspace_bytes);
+                     nullptr, true, workspace, workspace_bytes);
 }
 
 extern "C" int32_t nsg_linear_fp8_ws(const void* x, int64_t ldx, const void* w8, int64_t ldw8,
@@ -1044,7 +1052,7 @@ extern "C" int32_t nsg_linear_fp8_ws(const void* x, int64_t ldx, const void* w8,
                                      nsg_stream_t stream) {
   NSG_CHECK_ARG(w8 && w_scale, "null fp8 weight or scales");
   return linear_impl(x, ldx, nullptr, w8, ldw8, w_scale, bias, y, ldy, M, N, K, epilogue, stream,
-                     nullptr, workspace, workspace_bytes);
+                     nullptr, true, workspace, workspace_bytes);
 }
 
 extern "C" int32_t nsg_linear_rope_kv(const void* x, int64_t ldx, const void* w, int64_t ldw,

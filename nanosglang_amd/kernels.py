@@ -876,7 +876,7 @@ def silu_mul(gate_up: torch.Tensor, out: torch.Tensor | None = None) -> torch.Te
 
 
 LINEAR_BIAS, LINEAR_SILU_MUL = 0, 1
-SPLIT_K_MIN_WEIGHT = 16 << 20    # weights from which nsg_linear_workspace_bytes may be non-zero
+WS_FORM_MIN_WEIGHT = 16 << 20    # weights from which the *_ws entry points differ from the plain ones
 FP8 = torch.float8_e4m3fn
 
 
@@ -926,7 +926,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
            w_dequant: torch.Tensor | None = None, sumsq_in: torch.Tensor | None = None,
            norm_eps: float = 1e-6, residual: torch.Tensor | None = None,
            sumsq_out: torch.Tensor | None = None) -> torch.Tensor:
-    """y = x @ weight.T (+ bias) for bf16 (M, K) rows (C ABI: nsg_linear).
+    """y = x @ weight.T (+ bias) for bf16 (M, K) rows (C ABI: nsg_linear;
+    nsg_linear_ws for large weights without ``swiglu``).
 
     ``swiglu``: weight holds the fused [gate; up] rows (2I, K) and the
     result is bf16(silu(gate)) * up, (M, I).  ``weight`` may be
@@ -990,21 +991,20 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None = No
     if out is None:
         out = torch.empty(M, N, dtype=torch.bfloat16, device=x.device)
     epi = LINEAR_SILU_MUL if swiglu else LINEAR_BIAS
-    # large weights with few columns split K through fp32 partials: the
-    # caching allocator's memory, ordered with this stream's other work
-    need = 0 if swiglu or N * K < SPLIT_K_MIN_WEIGHT else \
-        lib.nsg_linear_workspace_bytes(M, N, K, epi)
-    if need > 0:
-        ws = torch.empty(need, dtype=torch.uint8, device=x.device)
+    if not swiglu and N * K >= WS_FORM_MIN_WEIGHT:
+        # large weights with few columns split K through fp32 partials: the
+        # caching allocator's memory, ordered with this stream's other work
+        need = lib.nsg_linear_workspace_bytes(M, N, K, epi)
+        ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need > 0 else None
         if fp8:
             check(lib.nsg_linear_fp8_ws(
                 x.data_ptr(), x.stride(0), weight.data_ptr(), weight.stride(0),
                 w_scale.data_ptr(), _ptr(bias), out.data_ptr(), out.stride(0), M, N, K, epi,
-                ws.data_ptr(), need, _stream_ptr(x.device)), "nsg_linear_fp8_ws")
+                _ptr(ws), need, _stream_ptr(x.device)), "nsg_linear_fp8_ws")
         else:
             check(lib.nsg_linear_ws(
                 x.data_ptr(), x.stride(0), weight.data_ptr(), weight.stride(0), _ptr(bias),
-                out.data_ptr(), out.stride(0), M, N, K, epi, ws.data_ptr(), need,
+                out.data_ptr(), out.stride(0), M, N, K, epi, _ptr(ws), need,
                 _stream_ptr(x.device)), "nsg_linear_ws")
         return out
     if fp8:
@@ -1030,9 +1030,11 @@ def linear_rope_kv(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | N
     """q/k/v projection + RoPE + KV-slot write (C ABI: nsg_linear_rope_kv, or
     nsg_linear_rope_kv_fp8 for float8_e4m3fn weights with per-row w_scale).
 
-    Same result as ``rope_kv_write(linear(x, weight, bias), ...)``; at row
-    counts where the library GEMM is the faster projection (prefill), or for
-    shapes the fused kernel does not take, it runs exactly that pair.
+    Same result as ``rope_kv_write(linear(x, weight, bias), ...)`` (bit for
+    bit with nsg_linear's projection; ``linear`` may add large weights up in
+    another order, nsg_linear_ws); at row counts where the library GEMM is the
+    faster projection (prefill), or for shapes the fused kernel does not take,
+    it runs exactly that pair.
     ``sumsq_in``: the folded RMSNorm's consumer side (nsg_linear_rope_kv_fold,
     see ``linear``; the fused kernel only).  Returns rotated q (M, Hq, D)."""
     _require_gpu(x, "x")

