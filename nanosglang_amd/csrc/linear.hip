@@ -784,29 +784,56 @@ using namespace nsg;
 constexpr int kFastRows = 160;
 constexpr int kFastRowsBig = 32;
 
-// Where ring_linear.hip takes over (both weight types alike, so that FP8 and
-// the bf16 weights it stands for agree bit for bit).  Graph replay, weights
-// cold, us, weight-streaming kernel -> ring:
-// * SwiGLU from 154 column tiles of 64 (enough workgroups for the GPU): 28672
-//   x 4096 FP8 30.3 -> 24.2 at 1 row, 39 -> 24.6 at 32, 57 -> 29.3 at 64, 108
-//   -> 58 at 160, bf16 43 -> 38 at 1 row; 22016 x 4096 FP8 24.9 -> 22.8 /
-//   47.9 -> 27.3 at 1 / 64; from 128 tiles above 32 rows (16384 x 4096: 32.9
-//   -> 27.1 at 64, but 19.6 -> 21.1 at 1; 8192 x 4096: 20.2 -> 26.4 at 64);
-// * bias, from 17 rows of weights of 24 M elements, K split: 4096 x 14336 FP8
-//   21.9 -> 16.8 at 17 rows, 34.5 -> 24.2 at 64, 63 -> 38 at 160 (14.5 ->
-//   17.6 at 16); 6144 x 4096 20.0 -> 17.3 at 64; 4096 x 4096 12.0 -> 14.8.
+// Where ring_linear.hip takes over.  Its workgroups take a CU each, so a grid a
+// little over a multiple of the CUs ends in a nearly empty round, and at few
+// rows short weights do not fill its ring.  Graph replay, weights cold, us,
+// weight-streaming kernel (bf16 SwiGLU from 33 rows: lm_head.hip's) -> ring:
+// * SwiGLU up to 32 rows: from 154 column tiles of 64 (28672 x 4096 FP8 30.3 ->
+//   24.2 at 1 row, 39 -> 24.6 at 32, bf16 43 -> 38 at 1; 16384 x 4096: 19.6 ->
+//   21.1 at 1), K from 2048 (20480 x 2 x 1024 FP8 12.8 -> 17.3), and more tiles
+//   than CUs only where the last round is more than three quarters full (17408
+//   x 2 x 5120, 272 tiles, bf16 75 -> 89 at 1 row);
+// * above 32 rows: from 128 tiles (16384 x 4096 FP8 32.9 -> 27.1 at 64 rows; 8192
+//   x 4096: 20.2 -> 26.4); past the CUs bf16 from a grid 19/32 full (16448 x 2 x
+//   4096, 257 tiles, 90 -> 100 at 129 rows, 19456 x 2 x 3072, 304 tiles, 96 ->
+//   83), FP8 there too if K is at least 2048 (257 tiles 119 -> 112);
+// * bias from 17 rows of weights of 24 M elements, K split over idle CUs: 4096 x
+//   14336 FP8 21.9 -> 16.8 at 17 rows, 34.5 -> 24.2 at 64, 63 -> 38 at 160 (14.5
+//   -> 17.6 at 16); 6144 x 4096 20.0 -> 17.3 at 64; 4096 x 4096 12.0 -> 14.8.
+//   Up to 32 rows K from 4096, or from 1024 with weights of 32 M (12288 x 2048
+//   bf16 13.2 -> 15.2 at 17 rows), and no nearly empty round (33280 x 4096, 260
+//   tiles, bf16 65 -> 70 at 17 rows); above 128 rows that only with K under 2048
+//   (33280 x 1024 FP8 38 -> 41 at 160 rows).
+// Up to 32 rows (SwiGLU) and throughout (bias) both weight types take the same
+// kernel, whose sums run in the same order for both: FP8 weights agree bit for
+// bit with the bf16 weights they stand for, unless the FP8 rows are 8- but not
+// 16-byte aligned (linear_impl): those stay on the weight-streaming kernel.
 constexpr int64_t kRingBiasWeight = 24ll << 20;
+constexpr int64_t kRingBiasWeightFew = 32ll << 20;
 constexpr int kRingBiasMinRows = 17;
+constexpr int kFewRows = 32;
+constexpr int kCus = 256;
 
-static bool ring_swiglu_big(int M, int N, int K) {
-  const int tiles = (N + 63) / 64;
-  return (int64_t)N * K >= kBigWeight && ring_linear_fits(M, N, K) &&
-         (tiles >= 154 || (tiles >= 128 && M > 32));
+// Workgroup slots of the rounds that `tiles` workgroups take.
+static int round_slots(int tiles) { return (tiles + kCus - 1) / kCus * kCus; }
+
+static bool ring_swiglu_big(int M, int N, int K, bool fp8) {
+  if ((int64_t)N * K < kBigWeight || !ring_linear_fits(M, N, K)) return false;
+  const int tiles = (N + 63) / 64, slots = round_slots(tiles);
+  if (M <= kFewRows)
+    return tiles >= 154 && K >= 2048 && (tiles <= kCus || 4 * tiles > 3 * slots);
+  return tiles >= 128 && (tiles <= kCus || 32 * tiles >= 19 * slots || (fp8 && K >= 2048));
 }
 
 static bool ring_bias_big(int M, int N, int K) {
-  return M >= kRingBiasMinRows && N < kWideN && (int64_t)N * K >= kRingBiasWeight &&
-         ring_linear_fits(M, N, K);
+  const int64_t weight = (int64_t)N * K;
+  if (M < kRingBiasMinRows || N >= kWideN || weight < kRingBiasWeight ||
+      !ring_linear_fits(M, N, K))
+    return false;
+  const int tiles = (N + 127) / 128;
+  const bool filled = tiles <= kCus || 32 * tiles >= 19 * round_slots(tiles);
+  if (M <= kFewRows) return filled && (K >= 4096 || (K >= 1024 && weight >= kRingBiasWeightFew));
+  return filled || K >= 2048 || M <= 128;
 }
 
 extern "C" int64_t nsg_linear_workspace_bytes(int32_t M, int32_t N, int32_t K,
@@ -932,7 +959,7 @@ int32_t linear_impl(const void* x, int64_t ldx, const void* w, const void* w8, i
   // *_ws entry points' only, so that nsg_linear stays nsg_linear_rope_kv's
   // projection bit for bit)
   if (!p.sumsq_in && !p.residual && (w || (ldw % 16 == 0 && (uintptr_t)w8 % 16 == 0)) &&
-      (silu ? ring_swiglu_big(M, N, K)
+      (silu ? ring_swiglu_big(M, N, K, !w)
             : ws_form && ring_bias_big(M, N, K) &&
                   (ring_ws == 0 || (workspace && workspace_bytes >= ring_ws &&
                                     (uintptr_t)workspace % 16 == 0)))) {

@@ -45,7 +45,8 @@ def test_swiglu_ragged_columns(M, I, K):
                                      (4100, 6400, 8), (33000, 768, 0)])
 def test_bias_split_k(M, N, K, pad):
     """pad 8: FP8 rows that are not 16-byte aligned stay on the weight-streaming
-    kernel; 33000 columns: K is not split."""
+    kernel; 33000 columns: K is not split, and up to 32 rows (its 258 column
+    tiles, K below 1024) the weight-streaming kernel is ahead."""
     print(f"case: bias {M} x {N} x {K}, row pad {pad}", flush=True)
     lib = _native.load()
     need = lib.nsg_linear_workspace_bytes(M, N, K, 0)
