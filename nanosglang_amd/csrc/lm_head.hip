@@ -44,13 +44,17 @@ namespace nsg {
 namespace {
 
 // Shapes of a workgroup (waves, columns per tile, row groups of waves).
-// * The argmax form: eight waves by 128 columns up to 80 rows and below 65536
-//   columns, ten by 160 otherwise (x is read once per tile: 13 % fewer bytes
-//   per CU), two row groups and column groups of 32 columns, so that a SIMD
-//   holds two or three waves.  Plain greedy call at 160 rows, us: four waves
-//   by 128 columns 67.2, eight 65.4, ten 63.6; 61.4 / 59.9 / 58.2 at 128 rows;
-//   at 32 ten waves are behind (folded call 52.5 against 51.3).  (From 65536
-//   columns a key per row and column group stays within 4 * ceil(N / 128).)
+// * The argmax form from 65536 columns and 65 rows on: ten waves by 160 columns,
+//   two row groups (x is read once per tile: 13 % fewer bytes per CU, and a SIMD
+//   holds two or three waves) where no workgroup walks more columns than with
+//   tiles of 128.  Folded call, tiles of 128 with four waves -> this, us:
+//   151,936 x 896 75.7 -> 70 at 160 rows, 200,000 x 512 67 -> 59; 128,256 x 896,
+//   four tiles of 160 against four of 128, 55 -> 65 at 112 rows.
+// * Otherwise tiles of 128: eight waves in two row groups at 33 - 64 rows (0.96
+//   of four waves over 14 weights) and from 97 (0.94 - 1.03); four waves at up to
+//   32 rows (eight: 1.01 - 1.02) and at 65 - 96, in two row groups (eight: 0.98
+//   - 1.12).  (From 65536 columns a key per row and column group stays within
+//   4 * ceil(N / 128).)
 // * The logits form: four waves by 128 columns; its stores set the pace, and
 //   with more waves a whole verify forward was 4 us slower (456 against 452).
 constexpr int kTenWaveMinN = 65536;
@@ -126,7 +130,7 @@ __global__ __launch_bounds__(kWaves * 64) void lm_head_kernel(HeadParams p) {
   // DMA sources.  Copy i of a wave fills ring slots (16-byte units) 64 i +
   // lane of its region: row r = slot / 8, physical segment slot % 8, which
   // holds logical segment (slot % 8) ^ ((r >> 1) & 7).  Rows past M repeat
-  // row M - 1, W rows past N repeat rows of the last four columns; their
+  // the first ones, W rows past N repeat rows of the last four columns; their
   // results are not kept.
   const uint32_t ring_lds = lds_addr(ring);
   const bf16* xsrc[kX];
@@ -138,7 +142,7 @@ __global__ __launch_bounds__(kWaves * 64) void lm_head_kernel(HeadParams p) {
     const int slot = copy * 64 + lane;
     const int r = slot >> 3;
     const int seg = (slot & 7) ^ ((r >> 1) & 7);
-    xsrc[i] = p.x + (int64_t)min(r, p.M - 1) * p.ldx + seg * 8;
+    xsrc[i] = p.x + (int64_t)(r % p.M) * p.ldx + seg * 8;
   }
   int wrow[kW], wseg[kW];
 #pragma unroll
@@ -579,11 +583,22 @@ int device_cus() {
   return cus[dev];
 }
 
+// Workgroups that walk N columns in tiles of COLS, and the columns that the
+// busiest of them walks.
+template <int MT, int COLS>
+int grid_of(int N) {
+  const int per_cu = kLdsMax / (ring_stages<MT, COLS>() * stage_bytes<MT, COLS>());
+  return std::min((N + COLS - 1) / COLS, device_cus() * std::max(per_cu, 1));
+}
+template <int MT, int COLS>
+int walked(int N) {
+  const int tiles = (N + COLS - 1) / COLS, grid = grid_of<MT, COLS>(N);
+  return (tiles + grid - 1) / grid * COLS;
+}
+
 template <int MT, int NW, int COLS, int RS, bool ARG>
 int32_t launch_shape(const HeadParams& p, hipStream_t s, int* key_cols) {
-  const int tiles = (p.N + COLS - 1) / COLS;
-  const int per_cu = kLdsMax / (ring_stages<MT, COLS>() * stage_bytes<MT, COLS>());
-  const int grid = std::min(tiles, device_cus() * std::max(per_cu, 1));
+  const int grid = grid_of<MT, COLS>(p.N);
   *key_cols = NW / RS * grid;
   if (p.sumsq)
     hipLaunchKernelGGL((lm_head_kernel<MT, NW, COLS, RS, ARG, true>), dim3(grid), dim3(NW * 64), 0,
@@ -598,9 +613,10 @@ template <int MT>
 int32_t launch_mt(const HeadParams& p, bool argmax, hipStream_t s, int* key_cols) {
   if (!argmax) return launch_shape<MT, 4, 128, MT >= 6 ? 2 : 1, false>(p, s, key_cols);
   if constexpr (MT >= 6) {
-    if (p.N >= kTenWaveMinN) return launch_shape<MT, 10, 160, 2, true>(p, s, key_cols);
+    if (p.N >= kTenWaveMinN && walked<MT, 160>(p.N) <= walked<MT, 128>(p.N))
+      return launch_shape<MT, 10, 160, 2, true>(p, s, key_cols);
   }
-  return launch_shape<MT, 8, 128, 2, true>(p, s, key_cols);
+  return launch_shape<MT, MT == 2 || MT == 6 ? 4 : 8, 128, MT == 2 ? 1 : 2, true>(p, s, key_cols);
 }
 
 template <int MT>

@@ -11,7 +11,7 @@ from nanosglang_amd import _native, kernels
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("M", [16, 80, 81, 96, 129, 160])
+@pytest.mark.parametrize("M", [1, 16, 33, 64, 65, 80, 81, 96, 97, 129, 160])
 @pytest.mark.parametrize("N", [4, 32, 164, 65532, 65536, 65700])
 def test_tokens_match_the_logits_form(M, N):
     print(f"case: {M} rows x {N} columns", flush=True)
