@@ -660,7 +660,7 @@ __global__ __launch_bounds__(kSThreads) void select_kernel(SmpParams p, bool vec
 // A row's K-th largest logit needs no histogram of the whole row: K of the
 // largest logits lie above the smallest of 16 numbers, wave w's ceil(K / 16)-th
 // largest lane maximum.  So one workgroup per row (1024 threads) reads the
-// row once -- bf16 rows of up to 155,648 logits stay in registers, longer and
+// row once -- bf16 rows of up to 155,640 logits stay in registers, longer and
 // fp32 rows are read a second time, from L2 --, collects the few hundred
 // logits at or above that bound in LDS, and evaluates the rule on them: the
 // K-th largest key by radix selection, then, over the tokens kept by top-k,
@@ -670,12 +670,13 @@ __global__ __launch_bounds__(kSThreads) void select_kernel(SmpParams p, bool vec
 // filter and three more, 7 - 10 us each whatever its work.  Eager calls, us,
 // staged -> this: 32 rows x 151,936 bf16, top-k 50 and top-p 0.9 57.2 -> 28.5,
 // top-k alone 41.3 -> 23.7, fp32 83 -> 41 / 56 -> 32; 32 x 32,000 bf16 41 -> 27;
-// top-k 200 and top-p 0.95 57 -> 39 (the sums over kept tokens grow with K^2:
-// the line lies at 256, where both forms are level).  About 10 us of that are
-// the marked rows' launches, which return at once.
+// top-k 200 and top-p 0.95 57 -> 39 (topk_ahead says where it is not ahead).
+// About 10 us of that are the marked rows' launches, which return at once.
 // Rows with so many ties that the lists overflow (more than 8192 logits at the
 // bound, or 1024 kept) are marked (todo), and the staged launches that follow do
-// those rows only: every other row's workgroups return at once.
+// those rows only: every other row's workgroups return at once.  Such rows pay
+// for both: 32 rows of one value, 151,936 bf16, top-k 50: 50 -> 69 us, with
+// top-p 0.9 78 -> 98.
 constexpr int kTkThreads = 1024;
 constexpr int kTkWaves = kTkThreads / 64;
 constexpr int kTkMaxK = 256;
@@ -963,10 +964,14 @@ __global__ __launch_bounds__(kTkThreads) void topk_kernel(SmpParams p) {
       if (__builtin_fmaf(v, p.c, -mc) >= -41.f) hi = mid;
       else lo = mid;
     }
+    if (hi <= bound) {  // nothing to leave out
+      if (tid == 0) p.todo[row] = 1;
+      return;
+    }
     __syncthreads();
     if (tid == 0) s_n = s_ns = 0;
     __syncthreads();
-    collect(max(bound, hi));
+    collect(hi);
     if (s_ns > kTkSlotCap || s_n > kTkCap) {
       if (tid == 0) p.todo[row] = 1;
       return;
@@ -1102,6 +1107,27 @@ __global__ __launch_bounds__(kTkThreads) void topk_kernel(SmpParams p) {
   }
 }
 
+// Where topk_kernel is ahead of the staged launches (graph replay, both sides,
+// 10 vocabularies of 1000 - 200,000, 1 - 1024 rows, eight settings): its
+// workgroups take a CU each and their sums grow with K^2, while the staged
+// launches grow with the elements.
+// * K to 128 (fp32, whose staged form has four levels a filter instead of two:
+//   200): 0.7 - 1.0 of the staged time at few elements, 0.26 at 128 x 151,936.
+//   More rows than CUs take a second round, which pays from about 8000 columns
+//   (512 x 1000 bf16, top-k 50: 26.5 -> 29 us; 1024 x 5000: 44 -> 62).
+// * K to 200 (fp32 256) from 2^20 elements: 1 x 128,256 bf16, top-k 200: 36 -> 37,
+//   16 x 128,256: 44 -> 38; K to 256 from 2^22 (4 x 151,936: 41 -> 51, 32 x
+//   151,936: 57 -> 52).
+bool topk_ahead(int rows, int V, int K, int esz) {
+  if (K <= 0 || K > kTkMaxK) return false;
+  constexpr int kCus = 256;
+  const int64_t elements = (int64_t)rows * V;
+  if (K <= (esz == 4 ? 200 : 128)) return rows <= kCus || V >= 8192;
+  if (K <= 200 || esz == 4)
+    return elements >= 1 << 20 && (rows <= kCus || V >= 16384);
+  return elements >= 1 << 22 && (rows <= kCus || V >= 32768);
+}
+
 struct SLayout {
   int nch, cs;
   int64_t cmax_off, hcnt_off, hmass_off, st_off, csum_off, ceq_off;
@@ -1219,7 +1245,7 @@ extern "C" int32_t nsg_sample(const void* logits, int64_t row_stride, int32_t lo
   p.csum = reinterpret_cast<u64*>(ws + L.csum_off);
   p.ceq = reinterpret_cast<uint32_t*>(ws + L.ceq_off);
   // (a workspace without room for the marks: the staged launches alone)
-  p.todo = p.K > 0 && p.K <= kTkMaxK && workspace_bytes >= L.total
+  p.todo = topk_ahead(rows, vocab, p.K, esz) && workspace_bytes >= L.total
                ? reinterpret_cast<uint32_t*>(ws + L.staged)
                : nullptr;
   const bool vec = (reinterpret_cast<uintptr_t>(logits) % 16 == 0) &&

@@ -43,6 +43,19 @@ def test_lengths_and_unaligned_rows(dtype, V):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("V", [155640, 160001])
+def test_many_kept(dtype, V):
+    """Top-k above 128: the one launch takes it from 2^20 elements (bf16 above 200,
+    2^22: 28 rows)."""
+    print(f"case: many kept, V {V} {dtype}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(V + 1)
+    x = torch.randn(28, V, generator=g, device="cuda").mul(2).to(dtype)
+    u = torch.rand(28, generator=g, device="cuda")
+    for K, P in ((129, 0.9), (200, 1.0), (256, 0.95), (256, 1.0)):
+        _check(x, 0.8, K, P, u)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 def test_ties_masks_and_signed_zeros(dtype):
     V = 20000
     g = torch.Generator(device="cuda").manual_seed(5)
