@@ -1142,7 +1142,7 @@ extern "C" int32_t nsg_linear_rope_kv_fold(
 extern "C" int64_t nsg_linear_argmax_workspace_bytes(int32_t M, int32_t N) {
   if (M <= 0 || N <= 0) return 0;
   // a key per 16 columns, and per column group of the lm_head kernel (up to 4
-  // in a single 128-column tile)
+  // in a single 128-column tile, which the folded form also takes for few columns)
   return (int64_t)M * std::max(4, (N + 15) / 16) * (int64_t)sizeof(uint64_t);
 }
 
@@ -1168,9 +1168,10 @@ extern "C" int32_t nsg_linear_argmax(const void* x, int64_t ldx, const void* w, 
                     (uintptr_t)w % 16 == 0 && (uintptr_t)bias % 8 == 0 &&
                     (uintptr_t)workspace % 8 == 0,
                 "x and w rows must be 16-byte aligned, bias and workspace 8-byte");
-  NSG_CHECK_ARG(workspace_bytes >= nsg_linear_argmax_workspace_bytes(M, N),
-                "workspace %lld bytes < %lld", (long long)workspace_bytes,
-                (long long)nsg_linear_argmax_workspace_bytes(M, N));
+  // (a key per 16 columns: the 4 keys of narrower outputs are the folded form's)
+  const int64_t need = (int64_t)M * ((N + 15) / 16) * (int64_t)sizeof(uint64_t);
+  NSG_CHECK_ARG(workspace_bytes >= need, "workspace %lld bytes < %lld",
+                (long long)workspace_bytes, (long long)need);
   LinParams p{};
   p.x = static_cast<const bf16*>(x);
   p.w = static_cast<const bf16*>(w);

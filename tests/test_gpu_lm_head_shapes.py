@@ -39,3 +39,23 @@ def test_tokens_match_the_logits_form(M, N):
         ws.data_ptr(), need, C.byref(kc), torch.cuda.current_stream().cuda_stream),
         "nsg_lm_head_fold_keys")
     assert kc.value <= 4 * -(-N // 128) and M * kc.value * 8 <= need
+
+
+@pytest.mark.parametrize("M,N", [(1, 4), (16, 32), (81, 48), (160, 20)])
+def test_plain_argmax_needs_one_key_per_16_columns(M, N):
+    """nsg_linear_argmax of few columns: its kernel writes a key per 16 columns, and
+    a workspace of that size (less than the folded form's) is enough."""
+    print(f"case: plain argmax, {M} rows x {N} columns", flush=True)
+    K = 256
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn(M, K, generator=g, device="cuda").bfloat16()
+    w = torch.randn(N, K, generator=g, device="cuda").bfloat16()
+    y = kernels.linear(x, w, force=True)
+    need = M * -(-N // 16) * 8
+    ws = torch.full((need + 4096,), 0x5A, dtype=torch.uint8, device="cuda")
+    tok = torch.empty(M, dtype=torch.int64, device="cuda")
+    kernels.check(_native.load().nsg_linear_argmax(
+        x.data_ptr(), K, w.data_ptr(), K, None, M, N, K, ws.data_ptr(), need, tok.data_ptr(), 1,
+        torch.cuda.current_stream().cuda_stream), "nsg_linear_argmax")
+    assert torch.equal(tok, (y == y.amax(-1, keepdim=True)).int().argmax(-1))
+    assert (ws[need:] == 0x5A).all()
