@@ -786,24 +786,25 @@ constexpr int kFastRowsBig = 32;
 
 // Where ring_linear.hip takes over.  Its workgroups take a CU each, so a grid a
 // little over a multiple of the CUs ends in a nearly empty round, and at few
-// rows short weights do not fill its ring.  Graph replay, weights cold, us,
-// weight-streaming kernel (bf16 SwiGLU from 33 rows: lm_head.hip's) -> ring:
-// * SwiGLU up to 32 rows: from 154 column tiles of 64 (28672 x 4096 FP8 30.3 ->
-//   24.2 at 1 row, 39 -> 24.6 at 32, bf16 43 -> 38 at 1; 16384 x 4096: 19.6 ->
-//   21.1 at 1), K from 2048 (20480 x 2 x 1024 FP8 12.8 -> 17.3), and more tiles
-//   than CUs only where the last round is more than three quarters full (17408
-//   x 2 x 5120, 272 tiles, bf16 75 -> 89 at 1 row);
-// * above 32 rows: from 128 tiles (16384 x 4096 FP8 32.9 -> 27.1 at 64 rows; 8192
-//   x 4096: 20.2 -> 26.4); past the CUs bf16 from a grid 19/32 full (16448 x 2 x
-//   4096, 257 tiles, 90 -> 100 at 129 rows, 19456 x 2 x 3072, 304 tiles, 96 ->
-//   83), FP8 there too if K is at least 2048 (257 tiles 119 -> 112);
+// rows short weights do not fill its ring.  Weights are named by rows x K.
+// Graph replay, weights cold, us, weight-streaming kernel (bf16 SwiGLU from 33
+// rows: lm_head.hip's) -> ring:
+// * SwiGLU up to 32 rows: from 154 column tiles of 64 (28672 x 4096 FP8 30 -> 26
+//   at 1 row, 41 -> 25 at 32, bf16 46 -> 42 at 1; 16384 x 4096: 19.6 -> 21.1 at 1),
+//   K from 2048 (40960 x 1024 FP8 12.8 -> 17.3), and more tiles than CUs only
+//   where the last round is more than three quarters full (34816 x 5120, 272
+//   tiles, bf16 75 -> 89 at 1 row);
+// * above 32 rows: from 128 tiles (16384 x 4096 FP8 35 -> 28 at 64 rows; 8192 x
+//   4096: 20.2 -> 26.4; 28672 x 4096 59 -> 30.5); past the CUs bf16 from a grid
+//   19/32 full (32896 x 4096, 257 tiles, 90 -> 100 at 129 rows; 38912 x 3072, 304
+//   tiles, 94 -> 82), FP8 there too if K is at least 2048 (257 tiles 119 -> 113);
 // * bias from 17 rows of weights of 24 M elements, K split over idle CUs: 4096 x
-//   14336 FP8 21.9 -> 16.8 at 17 rows, 34.5 -> 24.2 at 64, 63 -> 38 at 160 (14.5
-//   -> 17.6 at 16); 6144 x 4096 20.0 -> 17.3 at 64; 4096 x 4096 12.0 -> 14.8.
-//   Up to 32 rows K from 4096, or from 1024 with weights of 32 M (12288 x 2048
-//   bf16 13.2 -> 15.2 at 17 rows), and no nearly empty round (33280 x 4096, 260
-//   tiles, bf16 65 -> 70 at 17 rows); above 128 rows that only with K under 2048
-//   (33280 x 1024 FP8 38 -> 41 at 160 rows).
+//   14336 FP8 28 -> 18 at 17 rows, 44 -> 24 at 64, 75 -> 41 at 160; 6144 x 4096
+//   20.3 -> 17.3 at 64 (10.7 -> 12.2 at 8, 12.2 -> 12.6 at 16); 4096 x 4096 12.0
+//   -> 14.8.  Up to 32 rows K from 4096, or from 1024 with weights of 32 M (12288
+//   x 2048 bf16 13.2 -> 15.2 at 17 rows), and no nearly empty round (33280 x 4096,
+//   260 tiles, bf16 65 -> 70 at 17 rows); above 128 rows that only with K under
+//   2048 (33280 x 1024 FP8 38 -> 41 at 160 rows).
 // Up to 32 rows (SwiGLU) and throughout (bias) both weight types take the same
 // kernel, whose sums run in the same order for both: FP8 weights agree bit for
 // bit with the bf16 weights they stand for, unless the FP8 rows are 8- but not
@@ -894,7 +895,7 @@ int32_t apply_fold(LinParams& p, const NormFold* nf, int32_t N, bool consumer_ok
 }
 
 // Wide outputs (lm_head) without a bias or folded norm, bf16 weights:
-// lm_head.hip's kernel (x shared by 128 output columns), at any row count
+// lm_head.hip's kernel (x shared by 128 or 160 output columns), at any row count
 // for rows shorter than 2048 (151,936 x 896: 45 against 53 - 59 us at 1 - 32
 // rows), above 32 rows for longer ones (128,256 x 4096: there this kernel's
 // eight-tile shapes stream faster up to 32 rows, 177 against 198 us).

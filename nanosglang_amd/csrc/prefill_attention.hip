@@ -9,8 +9,8 @@
 // K or V fragment read from LDS feeds 32 rows instead of the verify kernel's
 // 16, and a workgroup of NW waves (32 NW rows of one request and KV head)
 // shares each K / V step, so LDS and L2 reads per flop are halved and
-// quartered.  No KV split: the planner takes this kernel only when the tiles
-// fill the GPU by themselves, so there is no merge launch either.
+// quartered.  No KV split: the planner takes this kernel only for enough well
+// filled tiles, so there is no merge launch either.
 //
 // Per workgroup, in 64-token steps through an LDS ring filled by DMA:
 //   * S^T = K Q^T (M = 32 tokens, N = 32 query rows): lane l holds row l % 32

@@ -29,7 +29,9 @@
 // 40 us (5.9 TB/s of weight; 68.6 before); FP8 29.3 us (57), where the chain of
 // a step -- LDS reads, conversion, MFMAs behind one barrier -- sets the pace,
 // not the stream: at 32 rows 24.6 us, and slots for more W in flight (x in a
-// shallow ring of its own) changed nothing at 64.
+// shallow ring of its own) changed nothing at 64.  (Torch callers reach the bf16
+// form at up to 32 rows: above, kernels.linear takes the library, with which it
+// has not been compared.)
 #include <algorithm>
 
 #include "lm_head.hpp"

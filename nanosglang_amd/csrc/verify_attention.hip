@@ -887,8 +887,8 @@ struct PrefillShape {
 // quarters) and there are enough of them: one workgroup per CU, or a third of
 // that with contexts of at most 2048 tokens.  256 rows only at head dim 128,
 // where two wave groups then alternate; at 64 the shorter 128-row workgroups
-// were ahead throughout (23.4 against 27.9 us on 32 prompts of 100 - 512
-// tokens); and not for four or more rounds of contexts up to 384 tokens, whose
+// were ahead throughout (by a sixth on 32 prompts of 100 - 512 tokens); and not
+// for four or more rounds of contexts up to 384 tokens, whose
 // few steps do not pay for the longer start (64 prompts of 128, 32 / 8 heads:
 // 256 rows 74 us, 128 rows 52, verify kernel 56).  From two workgroups per CU on
 // it is ahead; below, prefill_ahead decides.  Over 4,127 batches of nine head

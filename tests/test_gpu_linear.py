@@ -455,9 +455,9 @@ def test_fp8_linear_8b_shapes(M):
     """FP8 weights at the large shape's decoder linears (hidden 4096, 32 / 8
     heads of 128, FFN 14336): q/k/v 6144 x 4096 with RoPE + KV write, o_proj
     4096 x 4096, gate_up 28672 x 4096 with SwiGLU, down 4096 x 14336.  Each
-    is bit-exact against the bf16 kernel on the dequantised weights (the
-    weight-streaming kernel's 8B-class tile shapes, bf16 and FP8 alike) and
-    within bf16 rounding of an fp32 product."""
+    is bit-exact against the bf16 kernel on the dequantised weights (gate_up
+    above 32 rows within rounding, see _check_same_swiglu) and within bf16
+    rounding of an fp32 product."""
     from nanosglang_amd import kernels
     from nanosglang_amd.model.causal_lm import ModelConfig, rope_tables
     print(f"case: fp8 linear, 8B shapes, M={M}", flush=True)
