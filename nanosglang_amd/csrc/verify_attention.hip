@@ -921,11 +921,12 @@ PrefillShape prefill_shape(const int32_t* qo, const int32_t* kvp, int batch, int
 
 // Below two workgroups per CU the verify kernel's KV groups and splits can be
 // ahead, so both kernels' times are estimated (us, fitted to 3,890 batches of
-// nine head shapes, page size 16, each run on both: within 6 - 13 % rms).
-// Prefill: the start and the longest tile's 64-token steps, or all steps and
-// workgroups over the CUs.  Verify: with several KV groups the longest item's
-// 32-token steps per group and round, with one all steps over the CUs (or the
-// longest item), and the merge launch.  The prefill kernel is taken when its
+// nine head shapes at page size 16, and 440 of four at 1 and 4 for one KV
+// group, each run on both: within 6 - 14 % rms).  Prefill: the start and the
+// longest tile's 64-token steps, or all steps and workgroups over the CUs.
+// Verify: with several KV groups the longest item's 32-token steps per group
+// and round, with one all steps over the CUs (or half the longest item's), and
+// the merge launch.  The prefill kernel is taken when its
 // estimate is 10 % shorter (20 % for groups above 16, where the verify kernel's
 // tiles are as tall in both regimes).  Without the comparison 86 of the batches
 // were 3 - 77 % slower than on the verify kernel (16 x 16 query tokens over 600,
@@ -949,9 +950,12 @@ bool prefill_ahead(const PrefillShape& pre, int head_dim, int G, int num_cus, lo
     verify_us = head_dim == 64 ? 2.2 + 0.53 * sweep + 2.06 * rounds + (split ? 2.2 : 0.0)
                                : 2.6 + 0.78 * sweep + 2.5 * rounds + (split ? 1.9 : 0.0);
   } else {
-    const double sweep = std::max((double)longest_item, item_steps / cus);
-    verify_us = head_dim == 64 ? 19.6 + 0.289 * sweep + (split ? 7.4 : 0.0)
-                               : 29.3 + 0.516 * sweep + (split ? 10.8 : 0.0);
+    // few steps: a launch and the steps; many: the stream, with its own start
+    const double sweep = std::max(0.5 * longest_item, item_steps / cus);
+    verify_us = head_dim == 64 ? std::min(4.3 + 0.74 * sweep + (split ? 4.7 : 0.0),
+                                          19.6 + 0.286 * sweep + (split ? 8.6 : 0.0))
+                               : std::min(4.8 + 1.23 * sweep + (split ? 5.9 : 0.0),
+                                          30.1 + 0.508 * sweep + (split ? 12.9 : 0.0));
   }
   return prefill_us <= (G > 16 ? 0.8 : 0.9) * verify_us;
 }
@@ -1199,12 +1203,15 @@ int32_t plan_impl(const int32_t* qo_indptr_h, const int32_t* kv_indptr_h,
     // KV groups (one workgroup per CU): even shares when every workgroup runs
     // at once (level with chunks), and past that for two splits (48 rows over
     // 4000, 64 / 8 heads of 128: 92 in chunks, 66 in shares) or a rest of at
-    // most an eighth (128 over 4000, 16 / 2 heads: 63, 47); else whole chunks,
-    // whose rests free CUs early for the second round (48 over 1200, 32 / 32
-    // heads, 288 workgroups: 15.4 in chunks, 22.3 in shares).
+    // most an eighth with items behind it (128 over 4000, 16 / 2 heads: 63, 47;
+    // at the list's end the short rests are the second round: 64 over 2000, 32 /
+    // 32 heads: 25 in chunks, 31 in shares); else whole chunks, whose rests free
+    // CUs early for the second round (48 over 1200, 32 / 32 heads, 288
+    // workgroups: 15.4 in chunks, 22.3 in shares).
     const long long its = (g.kv_end + kTokIt - 1) / kTokIt;
     const long long rest = its - (ns - 1) * chunk_it;
-    const bool even = KS == 1 || all_at_once || ns == 2 || 8 * rest <= chunk_it;
+    const bool even = KS == 1 || all_at_once || ns == 2 ||
+                      (8 * rest <= chunk_it && oi + 1 < groups.size());
     auto cut = [&](int s) { return (even ? its * s / ns : s * chunk_it) * kTokIt; };
     for (int s = 0; s < ns; ++s) {
       int32_t* w = work_h + (size_t)n * NSG_ATTN_WORK_INTS;

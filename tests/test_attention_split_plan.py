@@ -29,6 +29,8 @@ CASES = [
     # splits or more: whole chunks and a rest
     ((48, 1200, 1, 32, 32, 128), 2, [16, 16, 5]),
     ((64, 16000, 1, 12, 12, 64), 4, [96, 96, 96, 96, 96, 19]),
+    # ... also with a rest of one step in the list's last tile
+    ((64, 2000, 1, 32, 32, 128), 2, [30, 31]),
     # ... two splits, or a rest of at most an eighth: even shares
     ((48, 4000, 1, 64, 8, 128), 2, None),
     ((128, 4000, 1, 16, 2, 128), 2, None),
@@ -54,6 +56,9 @@ def test_shares(case, groups, steps):
         assert all(a[1] == b[0] for a, b in zip(items, items[1:]))       # no gap, no overlap
         assert all(i[0] % 32 == 0 and i[2] == len(items) for i in items)
     first = [-(-(e - s) // 32) for s, e, _ in tiles[0]]
+    if L == 2000:
+        last = [-(-(e - s) // 32) for s, e, _ in list(tiles.values())[-1]]
+        assert last == [31, 31, 1]
     if steps is None:
         assert max(first) - min(first) <= 1
     else:

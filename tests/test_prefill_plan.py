@@ -121,3 +121,14 @@ def test_which_kernel_a_batch_gets(q, kv, heads, row_tiles):
     on both."""
     pl, _, _, _ = _plan(q, kv, *heads)
     assert pl.row_tiles == row_tiles if row_tiles else pl.row_tiles <= 4
+
+
+@pytest.mark.parametrize("P", [1, 4])
+@pytest.mark.parametrize("L,B,heads,prefill", [
+    (32, 16, (32, 8, 128), False), (100, 4, (32, 8, 128), False), (32, 32, (14, 2, 64), False),
+    (960, 1, (32, 8, 128), True), (256, 32, (14, 2, 64), True)])
+def test_small_pages_without_kv_groups(L, B, heads, prefill, P):
+    """Pages below 16 tokens: the verify kernel has one KV group only, which a few
+    short prompts still run faster on."""
+    pl, _, _, _ = _plan([L] * B, [L] * B, *heads, P=P)
+    assert (pl.row_tiles >= 8) == prefill
