@@ -1179,6 +1179,7 @@ int32_t plan_impl(const int32_t* qo_indptr_h, const int32_t* kv_indptr_h,
       order[(size_t)at[(size_t)(most - steps(groups[gi]))]++] = (int)gi;
   }
   const bool all_at_once = (long long)n * num_kv_heads <= num_cus;
+  const int most_splits = max_splits_planned(split_counts);
   n = 0;
   int m = 0;
   for (size_t oi = 0; oi < groups.size(); ++oi) {
@@ -1201,17 +1202,13 @@ int32_t plan_impl(const int32_t* qo_indptr_h, const int32_t* kv_indptr_h,
     // for a short rest lets the last workgroups end unevenly (large shape,
     // three draws of lengths: 308 / 302 / 298 -> 299 / 294 / 292 us).  Several
     // KV groups (one workgroup per CU): even shares when every workgroup runs
-    // at once (level with chunks), and past that for two splits (48 rows over
-    // 4000, 64 / 8 heads of 128: 92 in chunks, 66 in shares) or a rest of at
-    // most an eighth with items behind it (128 over 4000, 16 / 2 heads: 63, 47;
-    // at the list's end the short rests are the second round: 64 over 2000, 32 /
-    // 32 heads: 25 in chunks, 31 in shares); else whole chunks, whose rests free
-    // CUs early for the second round (48 over 1200, 32 / 32 heads, 288
-    // workgroups: 15.4 in chunks, 22.3 in shares).
+    // at once (level with chunks), and past that where no tile has more than
+    // two splits (48 rows over 4000, 64 / 8 heads of 128: 92 in chunks, 66 in
+    // shares); else whole chunks, whose rests free CUs early for the second
+    // round (48 over 1200, 32 / 32 heads, 288 workgroups: 15.4 in chunks, 22.3
+    // in shares; 64 over 2000: 25, 31).
     const long long its = (g.kv_end + kTokIt - 1) / kTokIt;
-    const long long rest = its - (ns - 1) * chunk_it;
-    const bool even = KS == 1 || all_at_once || ns == 2 ||
-                      (8 * rest <= chunk_it && oi + 1 < groups.size());
+    const bool even = KS == 1 || all_at_once || most_splits == 2;
     auto cut = [&](int s) { return (even ? its * s / ns : s * chunk_it) * kTokIt; };
     for (int s = 0; s < ns; ++s) {
       int32_t* w = work_h + (size_t)n * NSG_ATTN_WORK_INTS;

@@ -30,10 +30,9 @@ CASES = [
     ((48, 1200, 1, 32, 32, 128), 2, [16, 16, 5]),
     ((64, 16000, 1, 12, 12, 64), 4, [96, 96, 96, 96, 96, 19]),
     # ... also with a rest of one step in the list's last tile
-    ((64, 2000, 1, 32, 32, 128), 2, [30, 31]),
-    # ... two splits, or a rest of at most an eighth: even shares
+    ((64, 2000, 1, 32, 32, 128), 2, [31, 30]),
+    # ... no tile with more than two splits: even shares
     ((48, 4000, 1, 64, 8, 128), 2, None),
-    ((128, 4000, 1, 16, 2, 128), 2, None),
     # all workgroups at once: even shares
     ((64, 1100, 1, 14, 2, 64), 4, [16, 17]),
     # one KV group: even shares
