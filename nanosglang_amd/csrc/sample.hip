@@ -1118,10 +1118,14 @@ __global__ __launch_bounds__(kTkThreads) void topk_kernel(SmpParams p) {
 // * K to 200 (fp32 256) from 2^20 elements: 1 x 128,256 bf16, top-k 200: 36 -> 37,
 //   16 x 128,256: 44 -> 38; K to 256 from 2^22 (4 x 151,936: 41 -> 51, 32 x
 //   151,936: 57 -> 52).
-bool topk_ahead(int rows, int V, int K, int esz) {
+// * bf16 without top-p from 2^19: that staged form has five launches, and an
+//   eager call is bound by their number, one more here (2 x 128,256: 25.4 ->
+//   26.5 - 28.4, 4 x 151,936: 0.96 of the time; in a graph 0.8 - 0.9 at both).
+bool topk_ahead(int rows, int V, int K, int esz, bool top_p) {
   if (K <= 0 || K > kTkMaxK) return false;
   constexpr int kCus = 256;
   const int64_t elements = (int64_t)rows * V;
+  if (esz == 2 && !top_p && elements < 1 << 19) return false;
   if (K <= (esz == 4 ? 200 : 128)) return rows <= kCus || V >= 8192;
   if (K <= 200 || esz == 4)
     return elements >= 1 << 20 && (rows <= kCus || V >= 16384);
@@ -1245,7 +1249,7 @@ extern "C" int32_t nsg_sample(const void* logits, int64_t row_stride, int32_t lo
   p.csum = reinterpret_cast<u64*>(ws + L.csum_off);
   p.ceq = reinterpret_cast<uint32_t*>(ws + L.ceq_off);
   // (a workspace without room for the marks: the staged launches alone)
-  p.todo = topk_ahead(rows, vocab, p.K, esz) && workspace_bytes >= L.total
+  p.todo = topk_ahead(rows, vocab, p.K, esz, p.P < 1.0) && workspace_bytes >= L.total
                ? reinterpret_cast<uint32_t*>(ws + L.staged)
                : nullptr;
   const bool vec = (reinterpret_cast<uintptr_t>(logits) % 16 == 0) &&

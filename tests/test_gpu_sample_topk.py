@@ -38,7 +38,7 @@ def test_lengths_and_unaligned_rows(dtype, V):
     u = torch.rand(6, generator=g, device="cuda")
     for off in (0, 1, 3):                       # rows at every alignment
         x = base[:, off:off + V]
-        for K, P in ((1, 1.0), (8, 0.9), (50, 0.9), (256, 0.95), (257, 0.95)):
+        for K, P in ((1, 0.9), (1, 1.0), (8, 0.9), (50, 0.9), (128, 0.95), (256, 0.95), (257, 0.95)):
             _check(x, 0.8, K, P, u)
 
 
@@ -67,7 +67,7 @@ def test_ties_masks_and_signed_zeros(dtype):
     x[4, 1:] = x[4, 0] - 1                                   # one above them
     x[5] = torch.round(x[5] / 4)
     x = x.to(dtype)
-    for K, P in ((50, 0.9), (50, 1.0), (1, 0.5), (200, 0.99)):
+    for K, P in ((50, 0.9), (50, 1.0), (1, 0.5), (128, 0.95), (200, 0.99)):
         for u0 in (0.05, 0.37, 0.93):
             print(f"case: ties {dtype} K {K} P {P} u {u0}", flush=True)
             _check(x, 0.8, K, P, torch.full((8,), u0, device="cuda"))
